@@ -190,7 +190,8 @@ int mi_la_batch_host(const MiAlignParams *prm, const uint64_t *packed, long long
  * that does not fit gets status 6; tasks wider than the widest window keep
  * status 1 (window) or 2 (pool).  work (host, optional, 8 values): executed
  * band cells and snake compare steps, the aligner kernel time of each of the
- * 4 window levels in microseconds (HIP events on the launch stream), and the
+ * 4 levels (windows of 128, 256, 1,024 and 1,024 diagonals) in microseconds
+ * (HIP events on the launch stream), and the
  * number of task re-runs.  The library keeps its scratch between calls. */
 int mi_la_batch_device(const MiAlignParams *prm, const uint64_t *d_packed, long long npacked, const MiLaTask *d_tasks,
                        int ntasks, const int *d_order, MiLaResult *d_results, uint16_t *d_traces, long long trace_cap,
@@ -267,12 +268,12 @@ int mi_device_copy(void *dst, const void *src, long long bytes, int to_device);
 int mi_device_memset(void *p, int value, long long bytes);
 
 /* Launch shapes of the GPU kernels (no reference counterpart; results do
- * not depend on them): waves per CU of the report kernel's 64-diagonal
- * window (4..32, default 32) and of its 128-diagonal window (2..32, default
- * 16), the pebble pool of the 64-diagonal window as a power of two (12..18,
- * default 15), waves per CU of the batched aligner's 64-diagonal window
- * (4..32, default 32) and of its 128- and 256-diagonal windows (2..32,
- * default 16).  A 0 field keeps the default; NULL restores all defaults.
+ * not depend on them): waves per CU of the report kernel's first window
+ * (4..32, default 20; two pairs a wave) and of its 256-diagonal window (2..32,
+ * default 8), the pebble pool of the first window as a power of two (12..18,
+ * default 15), waves per CU of the batched aligner's first window (4..32,
+ * default 20) and of its 256-diagonal window (2..32, default 4).  A 0 field
+ * keeps the default; NULL restores all defaults.
  * The tuner in marvel_amd/tune.py picks them from a calibration run. */
 typedef struct {
     int report_waves_per_cu;

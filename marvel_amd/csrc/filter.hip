@@ -780,17 +780,6 @@ struct EvPair {
 };
 static EvPair g_ev_report, g_ev_sort;
 
-// The report kernel's first window for the next pass.  Every window computes
-// the same alignments, so this only decides speed: a pass that starts at 64
-// diagonals re-runs the pairs that outgrow them at 128 after a partial run,
-// which pays on blocks where few pairs do; on repeat-rich blocks, where the
-// 128-diagonal re-runs take longer than the whole 64-diagonal launch, the
-// next passes start at 128 (kReprobe of them, then one starts at 64 again to
-// re-measure).  Match_Filter runs one call at a time, as the reference's.
-static int g_report_first = 0, g_report_reprobe = 0;
-constexpr double kWideOverNarrow = 1.0;
-constexpr int kReprobe = 8;
-
 struct Level {
     int nch, pool_cap, mcap;
     long long mtcap;
@@ -1091,20 +1080,19 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
     const int w = maxdiag - mindiag + 1;
     const int maxtp_all = 2 * (std::max(A->maxlen, B->maxlen) / TS + 2);
     const int cus = mi_num_cus();
-    // waves per level: up to 8 per SIMD for the 64-window kernel; the per-wave
-    // pools are sized for typical pairs, outliers go to the larger levels
-    // aligner windows of 64, 128, 256 and 1,024 diagonals; the last level
-    // also has the large pebble pools and match arenas
-    constexpr int kLevels = 5;
+    // windows of 128 (a half's 30 diagonals, or the whole wave while a band is
+    // wider), 256 and 1,024 diagonals; the pools are sized for typical pairs,
+    // outliers go to the larger levels; the last also has the large pebble
+    // pools and match arenas
+    constexpr int kLevels = 4;
     const MiTuning& tu = mi_tuning();
-    const int l0_waves = cus * (tu.report_waves_per_cu ? tu.report_waves_per_cu : 32);
+    const int l0_waves = cus * (tu.report_waves_per_cu ? tu.report_waves_per_cu : 4 * kPackWaves);
     const int l0_pool = 1 << (tu.report_pool_log2 ? tu.report_pool_log2 : 15);
-    const int l1_waves = cus * (tu.report_l1_waves_per_cu ? tu.report_l1_waves_per_cu : 16);
-    const Level levels[kLevels] = {{1, l0_pool, 128, 1 << 16, l0_waves},
-                                   {2, 1 << 16, 256, 1 << 18, l1_waves},
-                                   {4, 1 << 17, 256, 1 << 18, cus * 8},
+    const int l1_waves = cus * (tu.report_l1_waves_per_cu ? tu.report_l1_waves_per_cu : 8);
+    const Level levels[kLevels] = {{2, l0_pool, 128, 1 << 16, l0_waves},
+                                   {4, 1 << 16, 256, 1 << 18, l1_waves},
                                    {16, 1 << 17, 256, 1 << 18, cus * 4},
-                                   {16, 1 << 20, 4096, 1LL << 22, std::min(cus, 256)}};
+                                   {16, 1 << 20, 4096, 1LL << 22, std::min(cus, 128)}};
     const int small_trace = TS <= TRACE_XOVR ? 1 : 0;
     const int tbytes = small_trace ? 1 : 2;
 
@@ -1255,7 +1243,6 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
     }
 
     int cur_level = -1, gen = 0;
-    double t_level[kLevels] = {0., 0., 0., 0., 0.};   // report kernel seconds per window of this pass
 
     // runs the n jobs listed at dorder (device) at `level`; returns the
     // (job, status) pairs that need another launch
@@ -1273,7 +1260,7 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
             mtrace.release();
             cur_level = level;
         }
-        const int gmax = L.waves;
+        const int gmax = 2 * (int)std::min<long long>(L.waves, std::max<long long>(n, nfirst));   // two pairs a wave
         bands.ensure((size_t)(3 * w + 2) * gmax);
         pools.ensure((size_t)L.pool_cap * gmax);
         pts.ensure((size_t)2 * 8192 * gmax);
@@ -1303,7 +1290,6 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
         b.otcap = otcap;
         g_ev_report.record_start();
         switch (L.nch) {
-        case 1: launch_report<1>(b, grid); break;
         case 2: launch_report<2>(b, grid); break;
         case 4: launch_report<4>(b, grid); break;
         default: launch_report<16>(b, grid); break;
@@ -1320,7 +1306,6 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
         const double sec = g_ev_report.seconds();
         S.t_report_kernel += sec;
         S.report_launches += 1;
-        t_level[level] += sec;
         u64 oc2[2];
         int nf = 0;
         HC(hipMemcpy(oc2, ocount.p, sizeof oc2, hipMemcpyDeviceToHost));
@@ -1361,11 +1346,10 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
 
     // runs a job list until every job is done: output-arena overflows are
     // re-run at the same window, wide bands / full pools at the next one.
-    // Jobs start at g_report_first; MI_REPORT_FIRST_LEVEL starts every job at
-    // the window it names instead (and keeps the choice fixed).
-    int first_level = g_report_first;
-    const char* fixed_first = getenv("MI_REPORT_FIRST_LEVEL");
-    if (fixed_first) first_level = std::min(std::max(atoi(fixed_first), 0), kLevels - 1);
+    // MI_REPORT_FIRST_LEVEL starts every job at the level it names.
+    int first_level = 0;
+    if (const char* e = getenv("MI_REPORT_FIRST_LEVEL"))
+        first_level = std::min(std::max(atoi(e), 0), kLevels - 1);
     auto run_all = [&](const int* dorder, long long n) {
         int level = first_level;
         std::vector<std::pair<int, int>> again = run(dorder, n, level);
@@ -1387,16 +1371,6 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
         }
     };
     run_all(order_all.p, nfirst);
-    if (!fixed_first) {
-        if (first_level == 0) {
-            if (t_level[0] > 0. && t_level[1] > kWideOverNarrow * t_level[0]) {
-                g_report_first = 1;
-                g_report_reprobe = kReprobe;
-            }
-        } else if (--g_report_reprobe <= 0) {
-            g_report_first = 0;
-        }
-    }
 
     // the cell shared by lastp[maxdiag] and lasta[mindiag-1] carries from
     // one pair to the next within a report chunk: re-run the pairs that

@@ -1,20 +1,20 @@
 // Batched Local_Alignment on gfx950: a persistent grid of single-wave
 // workgroups pulls alignment tasks from a device counter; every task is one
-// daligner Local_Alignment (dalign/align.c:1922-2060) computed by one wave64
-// (la_wave.hpp).
+// daligner Local_Alignment (dalign/align.c:1922-2060), computed by one half
+// of a wave64 (la_pack.hpp).
 //
 // Device-resident batch (mi_la_batch_device):
 //   * inputs stay in HBM: 2-bit packed reads and MiLaTask records;
 //   * each finished task reserves its A and B traces in a compact trace arena
 //     with one 64-bit atomic and copies them there, so the output is exactly
 //     the traces produced (no worst-case per-task slots, no clearing);
-//   * tasks that outgrow the 64-diagonal register window or the per-wave
-//     pebble pool append themselves to a device retry list and are re-run by
-//     a wider instantiation (128 / 256 / 1,024 diagonals, larger pools); only
-//     the retry count comes back to the host between levels;
+//   * tasks whose band outgrows the 128 diagonals of the first instantiation's
+//     wide window or their pebble pool append themselves to a device retry
+//     list and are re-run by a wider one (256 / 1,024 diagonals, larger
+//     pools); only the retry count comes back to the host between levels;
 //   * before a launch every task it covers is marked LA_UNRUN, so a launch
 //     stopped early (watchdog flag) can never leave a stale record behind;
-//   * the per-wave scratch (pebble pools, chain points, trace staging) is one
+//   * the scratch of each half (pebble pools, chain points, trace staging) is one
 //     workspace carved per level.  The library keeps a grown workspace per
 //     device, so repeated calls allocate nothing.
 #pragma once
@@ -24,16 +24,13 @@
 #include <cstdio>
 #include <cstring>
 
-#include "la_wave.hpp"
+#include "la_pack.hpp"
 #include "mi_common.h"
 
 namespace mi {
 
 constexpr int LA_SPACE = 6;   // the call's trace arena is full (task not written)
 constexpr int LA_UNRUN = 7;   // the launch stopped before reaching the task
-
-constexpr int kResInts = (int)(sizeof(MiLaResult) / sizeof(int));
-static_assert(sizeof(MiLaResult) == 80 && kResInts <= 64, "result record is written one int per lane");
 
 struct BatchScratch {
     Peb* pools;
@@ -44,88 +41,146 @@ struct BatchScratch {
     int latr_cap;
 };
 
+// Arguments of a launch, read through the kernarg segment.
+struct BatchArgs {
+    const MiLaTask* tasks;
+    const int* order;
+    int norder;
+    const uint64_t* pk;
+    DevSpec sp;
+    MiLaResult* res;
+    uint16_t* arena;
+    long long arena_cap;
+    unsigned long long* arena_top;
+    int* retry;
+    int* nretry;
+    BatchScratch ws;
+    int* counter;
+    unsigned long long* work;
+    const int* abort_flag;
+};
+
+// The tasks of a launch as the packed aligner's job (la_pack.hpp): half h of
+// workgroup b owns scratch slot 2 b + h.
+// (NCH: each kernel has its own copy, so its registers fit that kernel's.)
 template <int NCH>
-__global__ __launch_bounds__(64, NCH == 1 ? 8 : 1) void la_batch_kernel(
-    const MiLaTask* __restrict__ tasks, const int* __restrict__ order, int norder, const uint64_t* __restrict__ pk,
-    DevSpec sp, MiLaResult* __restrict__ res, uint16_t* __restrict__ arena, long long arena_cap,
-    unsigned long long* __restrict__ arena_top, int* __restrict__ retry, int* __restrict__ nretry, BatchScratch ws,
-    int* __restrict__ counter, unsigned long long* __restrict__ work, const int* abort_flag)
-{
-    const int wave = blockIdx.x;
-    const int lane = __lane_id();
-    Peb* pool = ws.pools + (size_t)wave * ws.pool_cap;
-    Peb* pts = ws.pts + (size_t)wave * 2 * ws.pts_cap;
-    uint16_t* latr = ws.latr + (size_t)wave * ws.latr_cap;
-    const int TS = sp.tspace;
-    long long tot_cells = 0, tot_snake = 0;
-    for (;;) {
-        // Every lane executes the atomic (only lane 0 adds 1), so no
-        // lane-dependent branch precedes the broadcast and the loop exit is
-        // wave-uniform; the first active lane is lane 0.
-        const int t = __builtin_amdgcn_readfirstlane(atomicAdd(counter, lane == 0 ? 1 : 0));
-        const int ab = __builtin_amdgcn_readfirstlane(__atomic_load_n(abort_flag, __ATOMIC_RELAXED));
-        if (t >= norder || ab) break;
-        const int ti = order ? order[t] : t;
-        const MiLaTask tk = tasks[ti];
-        const int mx = tk.alen > tk.blen ? tk.alen : tk.blen;
-        const int maxtp = 2 * (mx / TS + 2);
-        // Local_Alignment's borders (dalign/align.c:1966-1985): lbord/hbord < 0
-        // leave the wave unbounded, except that a read aligned to itself may not
-        // reach the main diagonal
-        const bool selfie = (tk.aword == tk.bword && tk.selfie);
-        const int minp = (tk.lbord < 0) ? ((selfie && tk.low >= 0) ? 1 : -INT32_MAX) : tk.low - tk.lbord;
-        const int maxp = (tk.hbord < 0) ? ((selfie && tk.hgh <= 0) ? -1 : INT32_MAX) : tk.hgh + tk.hbord;
-        WaveCount wc;
-        LaResult r;
-        if (4 * maxtp > ws.latr_cap) {
-            r.status = LA_POOL;
-        } else {
-            uint16_t* atr = latr + maxtp;
-            uint16_t* btr = latr + 3 * maxtp;
-            r = local_alignment<NCH>(sp, pk + tk.aword, tk.alen, pk + tk.bword, tk.blen, tk.comp, tk.low, tk.hgh,
-                                     tk.anti, minp, maxp, pool, ws.pool_cap, pts, ws.pts_cap, atr, btr, maxtp,
-                                     abort_flag, wc);
+struct BatchJob {
+    const BatchArgs* args;
+    int* ti;   // LDS: the task of each half
+
+    __device__ bool next(PackLds& L, int h)
+    {
+        const KernArgs<BatchArgs>* a = kern_args(args);
+        const int lane = __lane_id();
+        PackSlot& S = L.slot[h];
+        const int ab = uni(__atomic_load_n(a->abort_flag, __ATOMIC_RELAXED));
+        if (ab) return false;
+        // every lane executes the atomic (only lane 0 adds 1), so no lane-dependent branch precedes the broadcast
+        const int t = uni(atomicAdd(a->counter, lane == 0 ? 1 : 0));
+        if (t >= a->norder) return false;
+        const int i = a->order ? uni(a->order[t]) : t;
+        if (lane == 0) {
+            const MiLaTask tk = a->tasks[i];
+            const int slot = 2 * blockIdx.x + h;
+            const int TS = a->sp.tspace;
+            const int maxtp = 2 * ((tk.alen > tk.blen ? tk.alen : tk.blen) / TS + 2);
+            uint16_t* latr = a->ws.latr + (size_t)slot * a->ws.latr_cap;
+            // Local_Alignment's borders (dalign/align.c:1966-1985): lbord/hbord < 0
+            // leave the wave unbounded, except that a read aligned to itself may not
+            // reach the main diagonal
+            const bool selfie = (tk.aword == tk.bword && tk.selfie);
+            S.minp = (tk.lbord < 0) ? ((selfie && tk.low >= 0) ? 1 : -INT32_MAX) : tk.low - tk.lbord;
+            S.maxp = (tk.hbord < 0) ? ((selfie && tk.hgh <= 0) ? -1 : INT32_MAX) : tk.hgh + tk.hbord;
+            S.A = a->pk + tk.aword;
+            S.B = a->pk + tk.bword;
+            S.alen = tk.alen;
+            S.blen = tk.blen;
+            S.comp = tk.comp;
+            S.low = tk.low;
+            S.hgh = tk.hgh;
+            S.anti = tk.anti;
+            S.pool = a->ws.pools + (size_t)slot * a->ws.pool_cap;
+            S.pool_cap = 4 * maxtp > a->ws.latr_cap ? 0 : a->ws.pool_cap;   // 0: no room for the trace, LA_POOL
+            S.pts = a->ws.pts + (size_t)slot * 2 * a->ws.pts_cap;
+            S.pts_cap = a->ws.pts_cap;
+            S.atr = latr + maxtp;
+            S.btr = latr + 3 * maxtp;
+            S.maxtp = maxtp;
+            ti[h] = i;
         }
-        tot_cells += wc.cells;
-        tot_snake += wc.snake;
+        return true;
+    }
+
+    __device__ void done(PackLds& L, int h)
+    {
+        const KernArgs<BatchArgs>* a = kern_args(args);
+        const int lane = __lane_id();
+        PackSlot& S = L.slot[h];
+        const int i = uni(ti[h]);
+        int status = uni(S.res.status);
+        const int na = status == LA_OK ? uni(S.res.atlen) : 0, nb = status == LA_OK ? uni(S.res.btlen) : 0;
+        const int need = na + nb;
         long long off = 0;
-        int status = r.status;
         if (status == LA_OK) {
-            const int need = r.atlen + r.btlen;
-            unsigned long long o = atomicAdd(arena_top, lane == 0 ? (unsigned long long)need : 0ull);
-            off = (long long)__shfl(o, 0, 64);
-            if (off + need > arena_cap) {
+            const unsigned long long o = atomicAdd(a->arena_top, lane == 0 ? (unsigned long long)need : 0ull);
+            off = uni((long long)o);
+            if (off + need > a->arena_cap) {
                 status = LA_SPACE;
             } else {
-                const uint16_t* ta = latr + maxtp + r.afirst;
-                const uint16_t* tb = latr + 3 * maxtp + r.bfirst;
-                for (int i = lane; i < r.atlen; i += 64) arena[off + i] = ta[i];
-                for (int i = lane; i < r.btlen; i += 64) arena[off + r.atlen + i] = tb[i];
+                const uint16_t* ta = uni(S.atr) + uni(S.res.afirst);
+                const uint16_t* tb = uni(S.btr) + uni(S.res.bfirst);
+                uint16_t* out = a->arena + off;
+                for (int q = lane; q < na; q += 64) out[q] = ta[q];
+                for (int q = lane; q < nb; q += 64) out[na + q] = tb[q];
             }
         } else if (status == LA_WIDE || status == LA_POOL) {
-            const int q = __shfl(atomicAdd(nretry, lane == 0 ? 1 : 0), 0, 64);
-            if (lane == 0) retry[q] = ti;
+            const int q = uni(atomicAdd(a->nretry, lane == 0 ? 1 : 0));
+            if (lane == 0) a->retry[q] = i;
         }
-        const bool ok = status == LA_OK;
-        const int vals[kResInts] = {status,
-                                    ok ? r.abpos : 0, ok ? r.bbpos : 0, ok ? r.aepos : 0, ok ? r.bepos : 0,
-                                    ok ? r.diffs : 0,
-                                    ok ? r.b_abpos : 0, ok ? r.b_bbpos : 0, ok ? r.b_aepos : 0, ok ? r.b_bepos : 0,
-                                    ok ? r.atlen : 0, ok ? r.btlen : 0,
-                                    (int)(off & 0xffffffff), (int)(off >> 32),
-                                    (int)((off + (ok ? r.atlen : 0)) & 0xffffffff),
-                                    (int)((off + (ok ? r.atlen : 0)) >> 32),
-                                    (int)(wc.cells & 0xffffffff), (int)(wc.cells >> 32),
-                                    (int)(wc.snake & 0xffffffff), (int)(wc.snake >> 32)};
-        int v = 0;
-#pragma unroll
-        for (int q = 0; q < kResInts; q++) v = (lane == q) ? vals[q] : v;
-        if (lane < kResInts) reinterpret_cast<int*>(res + ti)[lane] = v;
+        if (lane == 0) {
+            MiLaResult r = {};
+            r.status = status;
+            if (status == LA_OK) {
+                r.abpos = S.res.abpos;
+                r.bbpos = S.res.bbpos;
+                r.aepos = S.res.aepos;
+                r.bepos = S.res.bepos;
+                r.diffs = S.res.diffs;
+                r.b_abpos = S.res.b_abpos;
+                r.b_bbpos = S.res.b_bbpos;
+                r.b_aepos = S.res.b_aepos;
+                r.b_bepos = S.res.b_bepos;
+                r.atlen = na;
+                r.btlen = nb;
+            }
+            r.atrace = off;
+            r.btrace = off + (status == LA_OK ? na : 0);
+            r.cells = S.cells;
+            r.snake = S.snake;
+            a->res[i] = r;
+            atomicAdd(&a->work[0], (unsigned long long)S.cells);
+            atomicAdd(&a->work[1], (unsigned long long)S.snake);
+        }
+        wave_sync();
     }
-    if (lane == 0) {
-        atomicAdd(&work[0], (unsigned long long)tot_cells);
-        atomicAdd(&work[1], (unsigned long long)tot_snake);
-    }
+};
+
+// A persistent grid of single-wave workgroups.  With a wave for every task
+// the upper halves stay idle.
+template <int NCH>
+__global__ __launch_bounds__(64, NCH == 2 ? kPackWaves : 1) void la_batch_kernel(BatchArgs)
+{
+    __shared__ PackLds L;
+    __shared__ int ti[2];
+    const BatchArgs* args = kernarg_ptr<BatchArgs>();
+    const KernArgs<BatchArgs>* a = kern_args(args);
+    DevSpec sp;
+    sp.table = a->sp.table;
+    sp.score = a->sp.score;
+    sp.tspace = a->sp.tspace;
+    sp.ave_path = a->sp.ave_path;
+    pack_tables(L, sp);
+    pack_run<NCH>(L, BatchJob<NCH>{args, ti}, a->norder > (int)gridDim.x, a->abort_flag);
 }
 
 // status of every task a launch covers := LA_UNRUN
@@ -164,6 +219,7 @@ struct Level {
     int pool_cap;
     int waves;   // upper bound; the scratch may cap it
 };
+constexpr int kSlots = 2;   // alignments a wave holds, each with its own scratch
 
 static const int kCounterBytes = 256;
 
@@ -174,7 +230,7 @@ static size_t wave_bytes(int pool_cap, int pts_cap, int latr_cap)
     return (size_t)pool_cap * sizeof(Peb) + (size_t)2 * pts_cap * sizeof(Peb) + (size_t)latr_cap * sizeof(uint16_t);
 }
 
-// carve `waves` waves of scratch at p (256-byte aligned pieces)
+// carve `waves` slots of scratch at p (256-byte aligned pieces)
 static BatchScratch carve(char* p, int waves, int pool_cap, int pts_cap, int latr_cap)
 {
     BatchScratch s;
@@ -203,25 +259,13 @@ static int launch_level(int nch, int grid, const MiLaTask* tasks, const int* ord
     if (hipMemsetAsync(counter, 0, sizeof(int), st) != hipSuccess) return -1;
     if (hipMemsetAsync(nretry, 0, sizeof(int), st) != hipSuccess) return -1;
     hipLaunchKernelGGL(k_la_mark_unrun, dim3((n + 255) / 256), dim3(256), 0, st, order, n, res);
+    const BatchArgs a{tasks, order, n, pk, sp, res, arena, arena_cap, arena_top, retry, nretry, ws, counter, work,
+                      abort_flag};
     switch (nch) {
-    case 1:
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<1>), dim3(grid), dim3(64), 0, st, tasks, order, n, pk, sp,
-                           res, arena, arena_cap, arena_top, retry, nretry, ws, counter, work, abort_flag);
-        break;
-    case 2:
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<2>), dim3(grid), dim3(64), 0, st, tasks, order, n, pk, sp,
-                           res, arena, arena_cap, arena_top, retry, nretry, ws, counter, work, abort_flag);
-        break;
-    case 4:
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<4>), dim3(grid), dim3(64), 0, st, tasks, order, n, pk, sp,
-                           res, arena, arena_cap, arena_top, retry, nretry, ws, counter, work, abort_flag);
-        break;
-    case 16:
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<16>), dim3(grid), dim3(64), 0, st, tasks, order, n, pk,
-                           sp, res, arena, arena_cap, arena_top, retry, nretry, ws, counter, work, abort_flag);
-        break;
-    default:
-        return -1;
+    case 2: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<2>), dim3(grid), dim3(64), 0, st, a); break;
+    case 4: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<4>), dim3(grid), dim3(64), 0, st, a); break;
+    case 16: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<16>), dim3(grid), dim3(64), 0, st, a); break;
+    default: return -1;
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -245,11 +289,11 @@ static BatchPlan make_plan(int maxlen, int tspace, int cus)
     p.latr_cap = 4 * (2 * (maxlen / tspace + 2));
     const int w0 = mi_tuning().batch_waves_per_cu;
     const int w1 = mi_tuning().batch_wide_waves_per_cu;
-    // windows of 64, 128, 256 and 1,024 diagonals; a task re-runs at the
+    // bands of up to 128, 256 and 1,024 diagonals; a task re-runs at the
     // next level when its band outgrows the window or its pool fills
-    p.lv[0] = Level{1, 1 << 15, cus * (w0 ? w0 : 32)};   // default 8 waves per SIMD
-    p.lv[1] = Level{2, 1 << 17, cus * (w1 ? w1 : 16)};
-    p.lv[2] = Level{4, 1 << 17, cus * (w1 ? w1 : 16)};
+    p.lv[0] = Level{2, 1 << 15, cus * (w0 ? w0 : 4 * kPackWaves)};
+    p.lv[1] = Level{4, 1 << 17, cus * (w1 ? w1 : 4)};
+    p.lv[2] = Level{16, 1 << 18, 256};
     p.lv[3] = Level{16, 1 << 20, 256};
     return p;
 }
@@ -311,16 +355,16 @@ static int run_batch(const DevSpec& sp, const uint64_t* pk, const MiLaTask* task
     int which = 0;
     for (int level = 0; level < 4 && n > 0; level++) {
         const Level& L = plan.lv[level];
-        const size_t per = wave_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap) + 3 * 256;
+        const size_t per = kSlots * wave_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap) + 3 * 256;
         long long g = std::min<long long>(L.waves, n);
         const long long fit = (area.bytes - fixed) / per;
         if (g > fit) g = fit;
-        while (g > 0 && carve_bytes((int)g, L.pool_cap, plan.pts_cap, plan.latr_cap) > area.bytes - fixed) g--;
+        while (g > 0 && carve_bytes(kSlots * (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap) > area.bytes - fixed) g--;
         if (g <= 0) {
             mi_set_error("batch: scratch too small for one wave of this level");
             return MI_ERR_ARG;
         }
-        const BatchScratch ws = carve(area.base + fixed, (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap);
+        const BatchScratch ws = carve(area.base + fixed, kSlots * (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap);
         int* retry = lists[which];
         if (work && hipEventRecord(ev[0], st) != hipSuccess) return MI_ERR_DEVICE;
         if (launch_level(L.nch, (int)g, tasks, cur, n, pk, sp, res, arena, arena_cap, d_arena_top, retry, ctr + 1, ws,

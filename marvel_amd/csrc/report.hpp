@@ -1,4 +1,5 @@
-// report_thread (dalign/filter.c:1617-1989) on gfx950: one wave per read pair.
+// report_thread (dalign/filter.c:1617-1989) on gfx950: one half-wave per read
+// pair while it aligns, the whole wave for what happens between alignments.
 //
 // The reference walks a pair's seeds (sorted by apos) in 50 kb panels that
 // overlap by 10 kb.  Per panel it scores diagonal bands (band = diag >> w),
@@ -6,17 +7,18 @@
 // score and the seed lies beyond the end of the last alignment that covered
 // its band (lasta).  Each alignment then raises lasta over its diagonal span.
 //
-// Here one wave owns the pair:
+// Here a half of a wave owns the pair (la_pack.hpp runs its alignments) and
+// the wave serves it in between:
 //   * band scores: 64 seeds at a time; lanes in the same band find each other
 //     with ballots, take the previous seed's apos from the lane below (or
 //     the band's lastp), add min(K, apos - prev) with atomics, and the last
 //     lane of the band stores lastp -- the order the sequential loop implies;
 //   * gating: the 64 seeds of a chunk test the condition together, the first
-//     passing lane is aligned by the whole wave (local_alignment), lasta is
-//     raised in parallel over the span, and testing resumes after that seed;
+//     passing lane is aligned, lasta is raised in parallel over the span, and
+//     testing resumes after that seed;
 //   * redundant alignments of the pair are fused by lane 0
 //     (dalign/filter.c:1249-1566) and the records are appended to the output.
-// The band arrays (score | lastp | lasta) of a wave use the reference's
+// The band arrays (score | lastp | lasta) of a half use the reference's
 // per-thread layout, so neighbour reads at the outer bands see the same
 // cells; any access outside [mindiag, maxdiag] is counted as an edge event.
 #pragma once
@@ -24,7 +26,7 @@
 #include <stdint.h>
 
 #include "filter_kernels.hpp"
-#include "la_wave.hpp"
+#include "la_pack.hpp"
 #include "records.h"
 
 namespace mi {
@@ -38,7 +40,7 @@ constexpr int RP_OUT = 5;      // output arena full (records not written)
 
 struct MPath {   // a kept alignment of the pair (dalign/align.h:76-83 fields)
     int tlen, diffs, abpos, bbpos, aepos, bepos;
-    long long toff;   // offset of its u16 trace in the wave's trace pool
+    long long toff;   // offset of its u16 trace in the half's trace pool
 };
 
 
@@ -58,17 +60,17 @@ struct ReportArgs {
     int K, binshift, hitmin, minhit, minover, tspace, small_trace;
     int mindiag, maxdiag, w;
     DevSpec sp;
-    // per-wave scratch
-    int* bands;         // (3w + 2) ints per wave, zero on entry, left zero on exit
+    // scratch of each half
+    int* bands;         // (3w + 2) ints, zero on entry, left zero on exit
     Peb* pools;
     int pool_cap;
     Peb* pts;
     int pts_cap;
-    uint16_t* latr;     // alignment trace scratch: 4 * maxtp_all per wave
+    uint16_t* latr;     // alignment trace scratch: 4 * maxtp_all
     int maxtp_all;
-    MPath* mpaths;      // 2 * mcap per wave (A list then B list)
+    MPath* mpaths;      // 2 * mcap (A list then B list)
     int mcap;
-    uint16_t* mtrace;   // mtcap per wave
+    uint16_t* mtrace;   // mtcap values
     long long mtcap;
     // the band cell shared by lastp[maxdiag] and lasta[mindiag-1]: its value
     // when the job starts (null: 0), at the end, and whether the job used it
@@ -244,149 +246,100 @@ __device__ int handle_redundancies(MPath* am, int n, MPath* bm, uint16_t* T, lon
 }
 
 // ---- the pair kernel --------------------------------------------------------------
-
-// The 64-lane window (NCH = 1) runs at 8 waves per SIMD (64 VGPRs, a few
-// spills): the aligner is bound by VALU issue and dependent latencies, and
-// measured on the 5 Mbp / 30x workload 3 -> 4 -> 5 -> 6 -> 8 waves per SIMD
-// took the kernel from 380 to 305, 277, 258 and 248 ms per step.
+//
 // AUX: the instantiation that also fills job_work / redund (capture mode and
-// the branch statistics); the default one keeps those pointers out of its
-// register budget.
-// The kernel's arguments read where they are used: a scalar load through the
-// kernarg segment pointer, made opaque to the compiler so that no argument is
-// held in (or spilled from) SGPRs across the aligner's loop.
-#ifndef MI_CPU_WAVE_EMU
-typedef const ReportArgs __attribute__((address_space(4))) KernArgs;
-__device__ __forceinline__ KernArgs* kargs()
-{
-    KernArgs* p = (KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return p;
-}
-#else
-// the CPU wave emulator (tests/wave_emu) hands the launch's arguments over
-typedef const ReportArgs KernArgs;
-inline KernArgs* kargs() { return (KernArgs*)emu::kernarg(); }
-#endif
-#define KA(f) (kargs()->f)
+// the branch statistics).
 
+// The pair a half works on, in LDS.
+struct PairState {
+    int active, in_panel, job, status;
+    long long ps, pe;        // its seeds
+    int ar, br, alen, blen, do_a, do_b;
+    int novla, novlb, tmin, tmax, touched, band0;
+    long long ttop, aligned, edges, cells, snake, steps;
+    long long lidx, nidx, h2, f0;   // panel [lidx, nidx), start of the next one, next seed to test
+    int amark2;
+};
+
+// (NCH: each kernel has its own copy, so its registers fit that kernel's)
 template <int NCH, bool AUX>
-__global__ __launch_bounds__(64, NCH == 1 ? 8 : 1) void k_report(ReportArgs)
-{
-    const int lane = __lane_id();
-    const int wave = blockIdx.x;
-    const int W3 = 3 * KA(w) + 2;
-    int* F = KA(bands) + (size_t)wave * W3;
-    int* score = F + 1 - KA(mindiag);             // score[band], band in [mindiag-1, maxdiag+1]
-    int* lastp = score + KA(w);
-    int* lasta = lastp + KA(w);
-    int* const edge = F + 2 * KA(w);              // lastp[maxdiag] == lasta[mindiag-1]
-    Peb* pool = KA(pools) + (size_t)wave * KA(pool_cap);
-    Peb* pts = KA(pts) + (size_t)wave * 2 * KA(pts_cap);
-    uint16_t* latr = KA(latr) + (size_t)wave * 4 * KA(maxtp_all);
-    MPath* am = KA(mpaths) + (size_t)wave * 2 * KA(mcap);
-    MPath* bm = am + KA(mcap);
-    uint16_t* T = KA(mtrace) + (size_t)wave * KA(mtcap);
-    const int TS = KA(tspace);
+struct PairJob {
+    const ReportArgs* args;
+    PairState* ps;   // LDS, one per half
 
-    for (;;) {
-        // all lanes take part in the atomic (lane 0 adds 1), so the loop exit is uniform
-        const int t = __builtin_amdgcn_readfirstlane(atomicAdd(KA(counter), lane == 0 ? 1 : 0));
-        const int ab = __builtin_amdgcn_readfirstlane(__atomic_load_n(KA(abort_flag), __ATOMIC_RELAXED));
-        if (t >= KA(norder) || ab) break;
-        const int job = KA(order)[t];
-        const int p = KA(jobs)[job];
-        const long long ps = KA(pstart)[p], pe = KA(pstart)[p + 1];
-        const int ar = KA(hits)[ps].aread, br = KA(hits)[ps].bread;
-        const int alen = KA(lenA)[ar], blen = KA(lenB)[br];
-        const uint64_t* Aseq = KA(pkA) + KA(w0A)[ar];
-        const uint64_t* Bseq = KA(pkB) + KA(w0B)[br];
-        const bool doA = alen >= KA(hgap_min);
-        const bool doB = KA(symmetric) && blen >= KA(hgap_min) && (ar != br || !KA(self) || !KA(comp));
-        const int maxtp = 2 * ((alen > blen ? alen : blen) / TS + 2);
-        uint16_t* atr = latr + maxtp;
-        uint16_t* btr = latr + 3 * maxtp;
-        int novla = 0, novlb = 0;
-        long long ttop = 0;
-        int pstatus = RP_OK;
-        int tmin = INT32_MAX, tmax = -INT32_MAX;   // lasta cells raised by this pair
-        bool touched = false;
-        long long aligned = 0, edges = 0;
-        WaveCount wc;
-        {
-            const int e0 = KA(edge_in) ? KA(edge_in)[job] : 0;
-            if (lane == 0) *edge = e0;
-            wave_sync();
-        }
+    typedef KernArgs<ReportArgs> KA;
 
-        long long nidx = ps;
-        int amark2 = 0;
-        while (nidx < pe && pstatus == RP_OK) {
-            const int amark = amark2 + 50000;
-            amark2 = amark - 10000;
-            const long long lidx = nidx;
-            // panel (dalign/filter.c:1740-1755): up to and including the first
-            // seed beyond amark; the next panel starts after the last seed at
-            // or before amark2
-            long long pend = pe, h2 = lidx;
-            for (long long c = lidx; c < pe; c += 64) {
-                const long long f = c + lane;
-                const int ap = (f < pe) ? KA(hits)[f].apos : INT32_MAX;
-                const unsigned long long beyond = __ballot(f < pe && ap > amark);
-                const unsigned long long within2 = __ballot(f < pe && ap <= amark2);
-                if (within2) h2 = c + highest_lane(within2) + 1;
-                if (beyond) {
-                    pend = c + lowest_lane(beyond) + 1;
-                    break;
+    struct Bands {
+        int *F, *score, *lastp, *lasta, *edge;
+    };
+    __device__ static Bands bands(KA* a, int slot)
+    {
+        // score[band], band in [mindiag-1, maxdiag+1]; edge: lastp[maxdiag] == lasta[mindiag-1]
+        Bands b;
+        b.F = a->bands + (size_t)slot * (3 * a->w + 2);
+        b.score = b.F + 1 - a->mindiag;
+        b.lastp = b.score + a->w;
+        b.lasta = b.lastp + a->w;
+        b.edge = b.F + 2 * a->w;
+        return b;
+    }
+
+    // the next alignment of half h: of its pair, or of the next pair in the queue
+    __device__ bool next(PackLds& L, int h)
+    {
+        KA* a = kern_args(args);
+        const int lane = __lane_id();
+        PairState& P = ps[h];
+        const int slot = 2 * blockIdx.x + h;
+        const Bands b = bands(a, slot);
+        for (;;) {
+            if (!uni(P.active)) {
+                // all lanes take part in the atomic (lane 0 adds 1), so the exit is uniform
+                const int t = uni(atomicAdd(a->counter, lane == 0 ? 1 : 0));
+                const int ab = uni(__atomic_load_n(a->abort_flag, __ATOMIC_RELAXED));
+                if (t >= a->norder || ab) return false;
+                if (lane == 0) {
+                    const int job = a->order[t], p = a->jobs[job];
+                    P.job = job;
+                    P.ps = a->pstart[p];
+                    P.pe = a->pstart[p + 1];
+                    const Seed s0 = a->hits[P.ps];
+                    P.ar = s0.aread;
+                    P.br = s0.bread;
+                    P.alen = a->lenA[s0.aread];
+                    P.blen = a->lenB[s0.bread];
+                    P.do_a = P.alen >= a->hgap_min;
+                    P.do_b = a->symmetric && P.blen >= a->hgap_min && (P.ar != P.br || !a->self || !a->comp);
+                    P.novla = P.novlb = 0;
+                    P.ttop = 0;
+                    P.status = RP_OK;
+                    P.tmin = INT32_MAX;   // lasta cells raised by this pair
+                    P.tmax = -INT32_MAX;
+                    P.touched = 0;
+                    P.aligned = P.edges = P.cells = P.snake = P.steps = 0;
+                    P.nidx = P.ps;
+                    P.amark2 = 0;
+                    P.in_panel = 0;
+                    P.active = 1;
+                    *b.edge = a->edge_in ? a->edge_in[job] : 0;
                 }
+                wave_sync();
             }
-            nidx = pend;
-            if (nidx - lidx >= KA(minhit)) {
-                // band scores (dalign/filter.c:1757-1766): each seed adds
-                // min(K, apos - apos of the band's previous seed)
-                for (long long c = lidx; c < nidx; c += 64) {
-                    const long long f = c + lane;
-                    const bool v = f < nidx;
-                    int ap = 0, band = KA(mindiag);
-                    if (v) {
-                        ap = KA(hits)[f].apos;
-                        band = KA(hits)[f].diag >> KA(binshift);
-                    }
-                    const unsigned bi = (unsigned)(band - KA(mindiag));
-                    unsigned long long peers = __ballot(v);
-#pragma unroll
-                    for (int b = 0; b < 16; b++) {
-                        const unsigned long long m = __ballot((bi >> b) & 1);
-                        peers &= ((bi >> b) & 1) ? m : ~m;
-                    }
-                    const unsigned long long below = peers & ((1ull << lane) - 1);
-                    const int prevl = below ? highest_lane(below) : lane;
-                    const int pap = __shfl(ap, prevl, 64);
-                    int prev = 0;
-                    if (v) prev = below ? pap : lastp[band];
-                    if (__any(v && band == KA(maxdiag))) touched = true;
-                    edges += __popcll(__ballot(v && (band == KA(mindiag) || band == KA(maxdiag))));
-                    wave_sync();
-                    if (v) {
-                        const int d = ap - prev;
-                        atomicAdd(&score[band], d >= KA(K) ? KA(K) : d);
-                        if (lane == highest_lane(peers)) lastp[band] = ap;
-                    }
-                    wave_sync();
-                }
+            const long long pe = uni(P.pe);
+            if (uni(P.in_panel)) {
                 // gating in seed order (dalign/filter.c:1768-1893): a seed is
                 // aligned when it lies beyond its band's lasta and the band
                 // pair score reaches hitmin; 64 seeds are tested at once and
                 // testing resumes after each aligned seed
-                long long f0 = lidx;
-                while (f0 < nidx && pstatus == RP_OK) {
+                const long long lidx = uni(P.lidx), nidx = uni(P.nidx);
+                long long f0 = uni(P.f0);
+                while (f0 < nidx && uni(P.status) == RP_OK) {
                     const long long f = f0 + lane;
-                    const bool v = f < nidx;
                     bool go = false;
-                    if (v) {
-                        const int ap = KA(hits)[f].apos, band = KA(hits)[f].diag >> KA(binshift);
-                        go = ap > lasta[band] && (score[band] + score[band + 1] >= KA(hitmin) ||
-                                                  score[band] + score[band - 1] >= KA(hitmin));
+                    if (f < nidx) {
+                        const int ap = a->hits[f].apos, band = a->hits[f].diag >> a->binshift;
+                        go = ap > b.lasta[band] && (b.score[band] + b.score[band + 1] >= a->hitmin ||
+                                                    b.score[band] + b.score[band - 1] >= a->hitmin);
                     }
                     const unsigned long long gm = __ballot(go);
                     if (!gm) {
@@ -394,140 +347,300 @@ __global__ __launch_bounds__(64, NCH == 1 ? 8 : 1) void k_report(ReportArgs)
                         continue;
                     }
                     const long long fh = f0 + lowest_lane(gm);
-                    f0 = fh + 1;
-                    const Seed sd = KA(hits)[fh];
-                    const int ap = sd.apos, dg = sd.diag, bp = ap - dg, band0 = dg >> KA(binshift);
-                    // a read against itself (-I, self forward pass: the same bases): the
-                    // wave may not reach the main diagonal (Local_Alignment's selfie
-                    // bounds, dalign/align.c:1966-1985)
-                    const bool selfie = KA(self) && !KA(comp) && ar == br;
-                    DevSpec spv;   // by value: the aligner reads the spec from SGPRs
-                    spv.table = KA(sp.table);
-                    spv.score = KA(sp.score);
-                    spv.tspace = KA(sp.tspace);
-                    spv.ave_path = KA(sp.ave_path);
-                    LaResult r = local_alignment<NCH>(spv, Aseq, alen, Bseq, blen, KA(comp), dg, dg, ap + bp,
-                                                      (selfie && dg >= 0) ? 1 : -INT32_MAX,
-                                                      (selfie && dg <= 0) ? -1 : INT32_MAX, pool, KA(pool_cap), pts,
-                                                      KA(pts_cap), atr, btr, maxtp, KA(abort_flag), wc);
-                    if (r.status != LA_OK) {
-                        pstatus = (r.status == LA_WIDE || r.status == LA_POOL || r.status == LA_ABORT) ? RP_RETRY
-                                                                                                        : RP_UNDEF;
-                        break;
+                    if (lane == 0) {
+                        const Seed sd = a->hits[fh];
+                        P.f0 = fh + 1;
+                        P.band0 = sd.diag >> a->binshift;
+                        align(L.slot[h], P, a, slot, sd);
                     }
-                    aligned++;
-                    const uint16_t* ta = atr + r.afirst;
-                    const uint16_t* tb = btr + r.bfirst;
-                    // Diagonal_Span (dalign/filter.c:1568-1599) widened by one
-                    // band on each side and to the seed's band
-                    int lo = r.abpos - r.bbpos, hi = lo;
-                    {
-                        int dd = r.aepos - r.bepos;
-                        if (dd < lo) lo = dd;
-                        else if (dd > hi) hi = dd;
-                        dd = (r.abpos / TS) * TS - r.bbpos;
-                        for (int i = 1; i < r.atlen - 2; i += 2) {   // same walk on every lane
-                            dd += TS - ta[i];
-                            if (dd < lo) lo = dd;
-                            else if (dd > hi) hi = dd;
-                        }
-                        lo = (lo >> KA(binshift)) - 1;
-                        hi = (hi >> KA(binshift)) + 1;
-                        if (band0 < lo) lo = band0;
-                        else if (band0 > hi) hi = band0;
-                    }
-                    if (lo < KA(mindiag) || hi > KA(maxdiag)) edges++;
-                    if (lo < KA(mindiag)) touched = true;
-                    // a consistent trace keeps the span within one band of the
-                    // array on each side; the clamp only guards the memory
-                    lo = max(lo, KA(mindiag) - 1);
-                    hi = min(hi, KA(maxdiag) + 1);
-                    tmin = min(tmin, lo);
-                    tmax = max(tmax, hi);
                     wave_sync();
-                    for (int i = lane; i <= hi - lo; i += 64)
-                        if (r.aepos > lasta[lo + i]) lasta[lo + i] = r.aepos;
-                    wave_sync();
-                    if ((r.aepos - r.abpos) + (r.bepos - r.bbpos) >= KA(minover)) {
-                        const long long need = (doA ? r.atlen : 0) + (doB ? r.btlen : 0);
-                        if (novla >= KA(mcap) || novlb >= KA(mcap) || ttop + need > KA(mtcap)) {
-                            pstatus = RP_ARENA;
-                            break;
-                        }
-                        if (doA) {
-                            for (int i = lane; i < r.atlen; i += 64) T[ttop + i] = ta[i];
-                            if (lane == 0)
-                                am[novla] = MPath{r.atlen, r.diffs, r.abpos, r.bbpos, r.aepos, r.bepos, ttop};
-                            ttop += r.atlen;
-                            novla++;
-                        }
-                        if (doB) {
-                            for (int i = lane; i < r.btlen; i += 64) T[ttop + i] = tb[i];
-                            if (lane == 0)
-                                bm[novlb] = MPath{r.btlen, r.diffs, r.b_abpos, r.b_bbpos, r.b_aepos, r.b_bepos, ttop};
-                            ttop += r.btlen;
-                            novlb++;
-                        }
-                        wave_sync();
-                    }
+                    return true;
                 }
                 // panel reset of the scored bands (dalign/filter.c:1895-1899)
                 wave_sync();
                 for (long long c = lidx; c < nidx; c += 64) {
                     const long long f = c + lane;
                     if (f < nidx) {
-                        const int band = KA(hits)[f].diag >> KA(binshift);
-                        score[band] = 0;
-                        lastp[band] = 0;
+                        const int band = a->hits[f].diag >> a->binshift;
+                        b.score[band] = 0;
+                        b.lastp[band] = 0;
                     }
+                }
+                if (lane == 0) {
+                    P.in_panel = 0;
+                    P.nidx = P.h2;
+                }
+                wave_sync();
+                continue;
+            }
+            const long long lidx = uni(P.nidx);
+            if (lidx < pe && uni(P.status) == RP_OK) {
+                panel(a, b, P, lidx, pe);
+                continue;
+            }
+            finish(a, b, P, slot);
+        }
+    }
+
+    // slot S's alignment of seed sd (lane 0)
+    __device__ static void align(PackSlot& S, const PairState& P, KA* a, int slot, const Seed& sd)
+    {
+        const int dg = sd.diag;
+        // a read against itself (-I, self forward pass: the same bases): the
+        // wave may not reach the main diagonal (Local_Alignment's selfie
+        // bounds, dalign/align.c:1966-1985)
+        const bool selfie = a->self && !a->comp && P.ar == P.br;
+        const int maxtp = 2 * ((P.alen > P.blen ? P.alen : P.blen) / a->tspace + 2);
+        uint16_t* latr = a->latr + (size_t)slot * 4 * a->maxtp_all;
+        S.A = a->pkA + a->w0A[P.ar];
+        S.B = a->pkB + a->w0B[P.br];
+        S.alen = P.alen;
+        S.blen = P.blen;
+        S.comp = a->comp;
+        S.low = S.hgh = dg;
+        S.anti = 2 * sd.apos - dg;
+        S.minp = (selfie && dg >= 0) ? 1 : -INT32_MAX;
+        S.maxp = (selfie && dg <= 0) ? -1 : INT32_MAX;
+        S.pool = a->pools + (size_t)slot * a->pool_cap;
+        S.pool_cap = a->pool_cap;
+        S.pts = a->pts + (size_t)slot * 2 * a->pts_cap;
+        S.pts_cap = a->pts_cap;
+        S.atr = latr + maxtp;
+        S.btr = latr + 3 * maxtp;
+        S.maxtp = maxtp;
+    }
+
+    // The panel from seed lidx on: its end, the next one's start, its band scores.
+    __device__ static void panel(KA* a, const Bands& b, PairState& P, long long lidx, long long pe)
+    {
+        const int lane = __lane_id();
+        const int amark = uni(P.amark2) + 50000, amark2 = amark - 10000;
+        // panel (dalign/filter.c:1740-1755): up to and including the first
+        // seed beyond amark; the next panel starts after the last seed at
+        // or before amark2
+        long long pend = pe, h2 = lidx;
+        for (long long c = lidx; c < pe; c += 64) {
+            const long long f = c + lane;
+            const int ap = (f < pe) ? a->hits[f].apos : INT32_MAX;
+            const unsigned long long beyond = __ballot(f < pe && ap > amark);
+            const unsigned long long within2 = __ballot(f < pe && ap <= amark2);
+            if (within2) h2 = c + highest_lane(within2) + 1;
+            if (beyond) {
+                pend = c + lowest_lane(beyond) + 1;
+                break;
+            }
+        }
+        const bool scored = pend - lidx >= a->minhit;
+        bool touched = false;
+        long long edges = 0;
+        if (scored) {
+            // band scores (dalign/filter.c:1757-1766): each seed adds
+            // min(K, apos - apos of the band's previous seed)
+            for (long long c = lidx; c < pend; c += 64) {
+                const long long f = c + lane;
+                const bool v = f < pend;
+                int ap = 0, band = a->mindiag;
+                if (v) {
+                    ap = a->hits[f].apos;
+                    band = a->hits[f].diag >> a->binshift;
+                }
+                const unsigned bi = (unsigned)(band - a->mindiag);
+                unsigned long long peers = __ballot(v);
+#pragma unroll
+                for (int q = 0; q < 16; q++) {
+                    const unsigned long long m = __ballot((bi >> q) & 1);
+                    peers &= ((bi >> q) & 1) ? m : ~m;
+                }
+                const unsigned long long below = peers & ((1ull << lane) - 1);
+                const int prevl = below ? highest_lane(below) : lane;
+                const int pap = __shfl(ap, prevl, 64);
+                int prev = 0;
+                if (v) prev = below ? pap : b.lastp[band];
+                if (__any(v && band == a->maxdiag)) touched = true;
+                edges += __popcll(__ballot(v && (band == a->mindiag || band == a->maxdiag)));
+                wave_sync();
+                if (v) {
+                    const int d = ap - prev;
+                    atomicAdd(&b.score[band], d >= a->K ? a->K : d);
+                    if (lane == highest_lane(peers)) b.lastp[band] = ap;
                 }
                 wave_sync();
             }
-            nidx = h2;
         }
+        if (lane == 0) {
+            P.amark2 = amark2;
+            P.lidx = lidx;
+            P.h2 = h2;
+            P.f0 = lidx;
+            P.in_panel = scored;
+            P.nidx = scored ? pend : h2;
+            if (touched) P.touched = 1;
+            P.edges += edges;
+        }
+        wave_sync();
+    }
+
+    // the alignment of half h ended (S.res)
+    __device__ void done(PackLds& L, int h)
+    {
+        KA* a = kern_args(args);
+        const int lane = __lane_id();
+        PairState& P = ps[h];
+        const PackSlot& S = L.slot[h];
+        const int slot = 2 * blockIdx.x + h;
+        const Bands b = bands(a, slot);
+        const int TS = a->tspace;
+        const int rs = uni(S.res.status);
+        if (lane == 0) {
+            P.cells += S.cells;
+            P.snake += S.snake;
+            P.steps += S.steps;
+        }
+        if (rs != LA_OK) {
+            if (lane == 0)
+                P.status = (rs == LA_WIDE || rs == LA_POOL || rs == LA_ABORT) ? RP_RETRY : RP_UNDEF;
+            wave_sync();
+            return;
+        }
+        const int abpos = uni(S.res.abpos), bbpos = uni(S.res.bbpos), aepos = uni(S.res.aepos),
+                  bepos = uni(S.res.bepos);
+        const int atlen = uni(S.res.atlen), btlen = uni(S.res.btlen);
+        const uint16_t* ta = uni(S.atr) + uni(S.res.afirst);
+        const uint16_t* tb = uni(S.btr) + uni(S.res.bfirst);
+        const int band0 = uni(P.band0);
+        // Diagonal_Span (dalign/filter.c:1568-1599) widened by one band on
+        // each side and to the seed's band.  The walk over the trace points is
+        // a prefix sum: 64 of them at a time.
+        int lo = abpos - bbpos, hi = lo;
+        {
+            const int d1 = aepos - bepos;
+            lo = min(lo, d1);
+            hi = max(hi, d1);
+            int dd = (abpos / TS) * TS - bbpos;
+            const int n = atlen / 2 - 1;   // every pair but the last
+            for (int c = 0; c < n; c += 64) {
+                const int i = c + lane;
+                int x = i < n ? TS - ta[2 * i + 1] : 0;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int u = __shfl_up(x, o, 64);
+                    if (lane >= o) x += u;
+                }
+                x += dd;
+                dd = rdl(x, 63);
+                int mn = i < n ? x : lo, mx = i < n ? x : hi;
+#pragma unroll
+                for (int o = 32; o >= 1; o >>= 1) {
+                    mn = min(mn, __shfl_xor(mn, o, 64));
+                    mx = max(mx, __shfl_xor(mx, o, 64));
+                }
+                lo = min(lo, uni(mn));
+                hi = max(hi, uni(mx));
+            }
+            lo = (lo >> a->binshift) - 1;
+            hi = (hi >> a->binshift) + 1;
+            if (band0 < lo) lo = band0;
+            else if (band0 > hi) hi = band0;
+        }
+        const bool out = lo < a->mindiag, over = out || hi > a->maxdiag;
+        // a consistent trace keeps the span within one band of the
+        // array on each side; the clamp only guards the memory
+        lo = max(lo, a->mindiag - 1);
+        hi = min(hi, a->maxdiag + 1);
+        for (int i = lane; i <= hi - lo; i += 64)
+            if (aepos > b.lasta[lo + i]) b.lasta[lo + i] = aepos;
+        const int do_a = uni(P.do_a), do_b = uni(P.do_b), na = uni(P.novla), nb = uni(P.novlb);
+        long long ttop = uni(P.ttop);
+        const bool keep = (aepos - abpos) + (bepos - bbpos) >= a->minover;
+        const long long need = (do_a ? atlen : 0) + (do_b ? btlen : 0);
+        const bool full = keep && (na >= a->mcap || nb >= a->mcap || ttop + need > a->mtcap);
+        MPath* am = a->mpaths + (size_t)slot * 2 * a->mcap;
+        MPath* bm = am + a->mcap;
+        uint16_t* T = a->mtrace + (size_t)slot * a->mtcap;
+        if (keep && !full) {
+            if (do_a) {
+                for (int i = lane; i < atlen; i += 64) T[ttop + i] = ta[i];
+                if (lane == 0) am[na] = MPath{atlen, S.res.diffs, abpos, bbpos, aepos, bepos, ttop};
+                ttop += atlen;
+            }
+            if (do_b) {
+                for (int i = lane; i < btlen; i += 64) T[ttop + i] = tb[i];
+                if (lane == 0)
+                    bm[nb] = MPath{btlen, S.res.diffs, S.res.b_abpos, S.res.b_bbpos, S.res.b_aepos, S.res.b_bepos, ttop};
+                ttop += btlen;
+            }
+        }
+        if (lane == 0) {
+            P.aligned += 1;
+            if (over) P.edges += 1;
+            if (out) P.touched = 1;
+            P.tmin = min(P.tmin, lo);
+            P.tmax = max(P.tmax, hi);
+            if (full) P.status = RP_ARENA;
+            else if (keep) {
+                P.novla = na + (do_a ? 1 : 0);
+                P.novlb = nb + (do_b ? 1 : 0);
+                P.ttop = ttop;
+            }
+        }
+        wave_sync();
+    }
+
+    // the pair is done: its records and statistics, its band arrays zero for the next one
+    __device__ static void finish(KA* a, const Bands& b, PairState& P, int slot)
+    {
+        const int lane = __lane_id();
+        const int job = uni(P.job), TS = a->tspace;
+        int pstatus = uni(P.status);
+        MPath* am = a->mpaths + (size_t)slot * 2 * a->mcap;
+        MPath* bm = am + a->mcap;
+        uint16_t* T = a->mtrace + (size_t)slot * a->mtcap;
         // per-pair lasta reset (dalign/filter.c:1905-1920): every raised cell
         // inside [mindiag, maxdiag] belongs to a run of non-zero cells through
         // a seed band of this pair, so the reference's walk clears exactly the
         // raised in-range cells; cells outside the range keep their value
+        const int tmin = uni(P.tmin), tmax = uni(P.tmax);
         if (tmin <= tmax) {   // some alignment raised cells (tmin / tmax start empty)
-            const int lo = max(tmin, KA(mindiag)), hi = min(tmax, KA(maxdiag));
-            for (int i = lane; i <= hi - lo; i += 64) lasta[lo + i] = 0;
+            const int lo = max(tmin, a->mindiag), hi = min(tmax, a->maxdiag);
+            for (int i = lane; i <= hi - lo; i += 64) b.lasta[lo + i] = 0;
             wave_sync();
         }
         if (pstatus == RP_OK) {
             // fuse redundant alignments (lane 0) and append the records
             bool ok = true;
-            int na = novla, nb = novlb;
-            if (lane == 0) {
+            int na = uni(P.novla), nb = uni(P.novlb);
+            if (lane == 0 && (AUX || na > 1 || nb > 1)) {
                 unsigned br[kRedundBranches] = {};
+                long long ttop = P.ttop;
+                const int comp = a->comp;
                 if (na > 1) {
-                    if (nb > 1) na = nb = handle_redundancies(am, na, bm, T, &ttop, KA(mtcap), TS, KA(comp), &ok, br);
-                    else na = handle_redundancies(am, na, nullptr, T, &ttop, KA(mtcap), TS, KA(comp), &ok, br);
+                    if (nb > 1) na = nb = handle_redundancies(am, na, bm, T, &ttop, a->mtcap, TS, comp, &ok, br);
+                    else na = handle_redundancies(am, na, nullptr, T, &ttop, a->mtcap, TS, comp, &ok, br);
                 } else if (nb > 1)
-                    nb = handle_redundancies(bm, nb, nullptr, T, &ttop, KA(mtcap), TS, KA(comp), &ok, br);
+                    nb = handle_redundancies(bm, nb, nullptr, T, &ttop, a->mtcap, TS, comp, &ok, br);
                 if constexpr (AUX) {
-                    if (KA(redund))   // the job's last successful run overwrites earlier ones
-                        for (int q = 0; q < kRedundBranches; q++) KA(redund)[(size_t)job * kRedundBranches + q] = br[q];
+                    if (a->redund)   // the job's last successful run overwrites earlier ones
+                        for (int q = 0; q < kRedundBranches; q++) a->redund[(size_t)job * kRedundBranches + q] = br[q];
                 }
             }
-            ok = __builtin_amdgcn_readfirstlane(ok ? 1 : 0) != 0;
-            na = __builtin_amdgcn_readfirstlane(na);
-            nb = __builtin_amdgcn_readfirstlane(nb);
+            ok = uni(ok ? 1 : 0) != 0;
+            na = uni(na);
+            nb = uni(nb);
             if (!ok) pstatus = RP_ARENA;
             else if (na + nb > 0) {
                 wave_sync();
                 long long tl = 0;
                 for (int i = 0; i < na; i++) tl += am[i].tlen;
                 for (int i = 0; i < nb; i++) tl += bm[i].tlen;
-                const int tbytes = KA(small_trace) ? 1 : 2;
-                unsigned long long r0 = 0, t0 = 0;
-                r0 = atomicAdd(&KA(ocount)[0], lane == 0 ? (unsigned long long)(na + nb) : 0ull);
-                t0 = atomicAdd(&KA(ocount)[1], lane == 0 ? (unsigned long long)(tl * tbytes) : 0ull);
-                const unsigned long long rbase = __shfl(r0, 0, 64);
-                const unsigned long long tbase = __shfl(t0, 0, 64);
-                if (rbase + na + nb > (unsigned long long)KA(ocap) || tbase + tl * tbytes > (unsigned long long)KA(otcap))
+                const int tbytes = a->small_trace ? 1 : 2;
+                const unsigned long long r0 = atomicAdd(&a->ocount[0], lane == 0 ? (unsigned long long)(na + nb) : 0ull);
+                const unsigned long long t0 = atomicAdd(&a->ocount[1], lane == 0 ? (unsigned long long)(tl * tbytes) : 0ull);
+                const unsigned long long rbase = (unsigned long long)uni((long long)r0);
+                const unsigned long long tbase = (unsigned long long)uni((long long)t0);
+                if (rbase + na + nb > (unsigned long long)a->ocap || tbase + tl * tbytes > (unsigned long long)a->otcap)
                     pstatus = RP_OUT;
                 else {
+                    const int ar = uni(P.ar) + a->afirst, br = uni(P.br) + a->bfirst;
                     unsigned long long to = tbase;
                     for (int i = 0; i < na + nb; i++) {
                         const bool isA = i < na;
@@ -540,23 +653,23 @@ __global__ __launch_bounds__(64, NCH == 1 ? 8 : 1) void k_report(ReportArgs)
                             o.bbpos = m.bbpos;
                             o.aepos = m.aepos;
                             o.bepos = m.bepos;
-                            o.flags = (uint32_t)KA(comp);
-                            o.aread = isA ? ar + KA(afirst) : br + KA(bfirst);
-                            o.bread = isA ? br + KA(bfirst) : ar + KA(afirst);
+                            o.flags = (uint32_t)a->comp;
+                            o.aread = isA ? ar : br;
+                            o.bread = isA ? br : ar;
                             o.local = isA ? i : i - na;
                             o.job = job;
                             o.toff = (long long)to;
-                            o.gen = KA(gen);
+                            o.gen = a->gen;
                             o.pad = 0;
-                            KA(orecs)[rbase + i] = o;
+                            a->orecs[rbase + i] = o;
                         }
                         // Compress_TraceTo8 (dalign/align.c:3352-3360) when the spacing is <= 125
                         for (int q = lane; q < m.tlen; q += 64) {
                             const uint16_t x = T[m.toff + q];
-                            if (tbytes == 1) KA(otr)[to + q] = (uint8_t)x;
+                            if (tbytes == 1) a->otr[to + q] = (uint8_t)x;
                             else {
-                                KA(otr)[to + 2 * q] = (uint8_t)(x & 0xff);
-                                KA(otr)[to + 2 * q + 1] = (uint8_t)(x >> 8);
+                                a->otr[to + 2 * q] = (uint8_t)(x & 0xff);
+                                a->otr[to + 2 * q + 1] = (uint8_t)(x >> 8);
                             }
                         }
                         to += (unsigned long long)m.tlen * tbytes;
@@ -565,35 +678,55 @@ __global__ __launch_bounds__(64, NCH == 1 ? 8 : 1) void k_report(ReportArgs)
             }
         }
         wave_sync();
-        const int eout = *edge;
+        const int eout = *b.edge;
         if (lane == 0) {
-            KA(status)[job] = pstatus;
-            if (pstatus == RP_OK) KA(final_gen)[job] = KA(gen);
-            KA(edge_out)[job] = eout;
-            KA(touch)[job] = touched ? 1 : 0;
+            a->status[job] = pstatus;
+            if (pstatus == RP_OK) a->final_gen[job] = a->gen;
+            a->edge_out[job] = eout;
+            a->touch[job] = P.touched;
             if (pstatus == RP_OK) {
-                atomicAdd(&KA(stats)[0], (unsigned long long)aligned);
-                atomicAdd(&KA(stats)[1], (unsigned long long)wc.cells);
-                atomicAdd(&KA(stats)[2], (unsigned long long)wc.snake);
-                atomicAdd(&KA(stats)[3], (unsigned long long)edges);
-                atomicAdd(&KA(stats)[4], (unsigned long long)wc.steps);
+                atomicAdd(&a->stats[0], (unsigned long long)P.aligned);
+                atomicAdd(&a->stats[1], (unsigned long long)P.cells);
+                atomicAdd(&a->stats[2], (unsigned long long)P.snake);
+                atomicAdd(&a->stats[3], (unsigned long long)P.edges);
+                atomicAdd(&a->stats[4], (unsigned long long)P.steps);
                 if constexpr (AUX) {
-                    if (KA(job_work)) KA(job_work)[job] = (unsigned long long)(wc.cells + wc.snake);
+                    if (a->job_work) a->job_work[job] = (unsigned long long)(P.cells + P.snake);
                 }
             }
         }
         // leave the band arrays zero for the next job: the edge cell and the
         // pad always, everything when the pair stopped early
+        const int W3 = 3 * a->w + 2;
         if (pstatus != RP_OK) {
             wave_sync();
-            for (int i = lane; i < W3; i += 64) F[i] = 0;
+            for (int i = lane; i < W3; i += 64) b.F[i] = 0;
         } else if (lane == 0) {
-            *edge = 0;
-            F[W3 - 1] = 0;
+            *b.edge = 0;
+            b.F[W3 - 1] = 0;
         }
+        if (lane == 0) P.active = 0;
         wave_sync();
     }
+};
+
+// A persistent grid of single-wave workgroups, two pairs in flight on each
+// (one where the grid has a wave for every pair).
+template <int NCH, bool AUX>
+__global__ __launch_bounds__(64, NCH == 2 ? kPackWaves : 1) void k_report(ReportArgs)
+{
+    __shared__ PackLds L;
+    __shared__ PairState ps[2];
+    const ReportArgs* args = kernarg_ptr<ReportArgs>();
+    KernArgs<ReportArgs>* a = kern_args(args);
+    if (__lane_id() < 2) ps[__lane_id()].active = 0;
+    DevSpec sp;
+    sp.table = a->sp.table;
+    sp.score = a->sp.score;
+    sp.tspace = a->sp.tspace;
+    sp.ave_path = a->sp.ave_path;
+    pack_tables(L, sp);
+    pack_run<NCH>(L, PairJob<NCH, AUX>{args, ps}, a->norder > (int)gridDim.x, a->abort_flag);
 }
-#undef KA
 
 }  // namespace mi

@@ -66,6 +66,76 @@ __global__ __launch_bounds__(64) void st_match(const uint64_t* A, const uint64_t
     out[2 * i + 1] = mism ? 1 : 0;
 }
 
+// value of lane (L-1) & 63 / (L+1) & 63: DPP wave_ror:1 / wave_rol:1, full-rate
+// VALU moves (no LDS traffic).  All 64 lanes must be active.
+// (every lane has a source, so no "old" value is needed: one v_mov_b32_dpp)
+__device__ __forceinline__ int lane_below(int v) { return __builtin_amdgcn_mov_dpp(v, 0x13C, 0xF, 0xF, false); }
+__device__ __forceinline__ int lane_above(int v) { return __builtin_amdgcn_mov_dpp(v, 0x134, 0xF, 0xF, false); }
+// Wave-wide scans from DPP row moves (no LDS): row_shl:n / row_shr:n read
+// lane L+n / L-n of the same 16-lane row, row_bcast:15 / :31 hand the last
+// lane of a row (of two rows) to the next row(s).  Lanes without a source
+// read 0 (bound_ctrl), the identity of max over non-negative values, so each
+// level is a single v_max_i32 with a DPP operand.
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ int dpp0(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xF, true);
+}
+// inclusive max over lanes >= L of x >= 0
+__device__ __forceinline__ int suffix_max_nn(int x)
+{
+    x = max(x, dpp0<0x101>(x));   // row_shl:1
+    x = max(x, dpp0<0x102>(x));   // row_shl:2
+    x = max(x, dpp0<0x104>(x));   // row_shl:4
+    x = max(x, dpp0<0x108>(x));   // row_shl:8
+    // lane 16r now holds row r's maximum; lanes of row r add the rows above
+    // it, selected with arithmetic masks (-1 / 0) rather than lane masks
+    const int s1 = __builtin_amdgcn_readlane(x, 16), s2 = __builtin_amdgcn_readlane(x, 32);
+    const int s3 = __builtin_amdgcn_readlane(x, 48);
+    int row = __lane_id() >> 4;
+    asm volatile("" : "+v"(row));   // keeps the row masks from being hoisted into (spilled) SGPR lane masks
+    const int m1 = (row - 1) >> 31, m2 = (row - 2) >> 31, m3 = (row - 3) >> 31;
+    return max(max(x, s1 & m1), max(s2 & m2, s3 & m3));
+}
+// inclusive max over lanes <= L of x >= 0
+__device__ __forceinline__ int prefix_max_nn(int x)
+{
+    x = max(x, dpp0<0x111>(x));        // row_shr:1
+    x = max(x, dpp0<0x112>(x));        // row_shr:2
+    x = max(x, dpp0<0x114>(x));        // row_shr:4
+    x = max(x, dpp0<0x118>(x));        // row_shr:8
+    x = max(x, dpp0<0x142, 0xA>(x));   // row_bcast:15 into rows 1, 3
+    x = max(x, dpp0<0x143, 0xC>(x));   // row_bcast:31 into rows 2, 3
+    return x;
+}
+// value of lane L+1 / L-1; the lane without one (63 / 0) gets `edge`
+// (DPP wave_shl:1 / wave_shr:1)
+__device__ __forceinline__ int lane_above_or(int v, int edge) { return __builtin_amdgcn_update_dpp(edge, v, 0x130, 0xF, 0xF, false); }
+__device__ __forceinline__ int lane_below_or(int v, int edge) { return __builtin_amdgcn_update_dpp(edge, v, 0x138, 0xF, 0xF, false); }
+// inclusive max over lanes >= L (x >= -1).  GATHER: the lanes reversed by one
+// ds_bpermute each way around the DPP prefix scan, for passes that run many
+// waves per SIMD (the LDS pipe is idle there, the VALU is not); otherwise
+// the DPP suffix scan, which keeps the two LDS round trips off the path of a
+// wave that runs alone (the wider windows).
+template <bool GATHER>
+__device__ __forceinline__ int wave_suffix_max(int x)
+{
+    if constexpr (GATHER) {
+        const int r = 63 - __lane_id();
+        return __shfl(prefix_max_nn(__shfl(x + 1, r, 64)), r, 64) - 1;
+    } else {
+        return suffix_max_nn(x + 1) - 1;
+    }
+}
+// inclusive min over lanes <= L (any x): the max of INT32_MAX - x >= 0
+__device__ __forceinline__ int wave_prefix_min(int x) { return 2147483647 - prefix_max_nn(2147483647 - x); }
+
+// fields of lane L + sel (sel in {-1, 0, +1}, wrapping like (L + sel) & 63)
+__device__ __forceinline__ int pick3(int v, int sel)
+{
+    const int b = lane_below(v), a = lane_above(v);
+    return sel < 0 ? b : (sel > 0 ? a : v);
+}
 // test 3: DPP lane moves; per lane: [lane_below(v), lane_above(v), the
 // scans, the edge moves, the DPP suffix max, pick3 with sel = L % 3 - 1]
 __global__ __launch_bounds__(64) void st_dpp(const int* in, int* out)

@@ -1,8 +1,8 @@
 """Autotuner of the GPU launch shapes (no reference counterpart).
 
-The report kernel's waves per CU at the 64- and 128-diagonal windows, the
-pebble pool of the 64-diagonal window and the batched aligner's waves per CU
-at its 64-diagonal and its wider windows (MiTuning, include/marvl_align.h)
+The report kernel's waves per CU at its first and its 256-diagonal window,
+the pebble pool of the first window and the batched aligner's waves per CU at
+its first and its 256-diagonal window (MiTuning, include/marvl_align.h)
 change how fast a pass runs, never what it writes.  The tuner times short calibration runs of the caller's own
 workload with each candidate, keeps the fastest, and stores the choice per
 device (architecture and compute units) in a JSON cache, so later processes
@@ -22,13 +22,13 @@ from .lib import MiTuning, lib
 
 FIELDS = ("report_waves_per_cu", "report_pool_log2", "report_l1_waves_per_cu", "batch_waves_per_cu",
           "batch_wide_waves_per_cu")
-DEFAULT = {"report_waves_per_cu": 32, "report_pool_log2": 15, "report_l1_waves_per_cu": 16, "batch_waves_per_cu": 32,
-           "batch_wide_waves_per_cu": 16}
-REPORT_CANDIDATES = [(w, p) for w in (16, 24, 32) for p in (14, 15, 16)]
-L1_CANDIDATES = (8, 16, 24, 32)
-# (64-diagonal window, wider windows): the levels are timed apart, so each
+DEFAULT = {"report_waves_per_cu": 20, "report_pool_log2": 15, "report_l1_waves_per_cu": 8, "batch_waves_per_cu": 20,
+           "batch_wide_waves_per_cu": 4}
+REPORT_CANDIDATES = [(w, p) for w in (12, 16, 20) for p in (14, 15)]
+L1_CANDIDATES = (4, 8, 12)
+# (first window, 256-diagonal window): the levels are timed apart, so each
 # run scores one candidate of each and the two are chosen independently
-BATCH_CANDIDATES = ((16, 8), (24, 12), (32, 16), (32, 20))
+BATCH_CANDIDATES = ((16, 2), (20, 4), (24, 8))
 
 
 def cache_path() -> str:
@@ -91,8 +91,7 @@ def _time_report(step, reps=1) -> float:
 
 class _FirstLevel:
     """Pins the report kernel's first window (MI_REPORT_FIRST_LEVEL) for a
-    calibration loop, so the library's own choice of it does not move
-    between candidates."""
+    calibration loop."""
 
     def __init__(self, level: int):
         self.level = str(level)
@@ -112,13 +111,10 @@ class _FirstLevel:
 def tune_report(step) -> dict:
     """Picks the report kernel's shapes with `step()` (one block-pair
     comparison returning both passes' stats): waves per CU and pool at the
-    64-diagonal window, then waves per CU at the 128-diagonal window.  The
-    latter are timed with every pair started at the 128-diagonal window
-    (MI_REPORT_FIRST_LEVEL=1): in an ordinary step that window re-runs only
-    the few pairs that outgrow 64 diagonals, which no candidate changes
-    measurably, while on repeat-rich blocks it carries as much work as the
-    64-diagonal window and the shape matters (8 waves per CU ran 19 % slower
-    than 16 to 32 there)."""
+    first window, then waves per CU at the 256-diagonal window.  The latter
+    are timed with every pair started there (MI_REPORT_FIRST_LEVEL=1): in an
+    ordinary step that window re-runs only the few pairs that outgrow 128
+    diagonals, which no candidate changes measurably."""
     base = current()
     timings = {}
     with _FirstLevel(0):
@@ -139,7 +135,7 @@ def tune_report(step) -> dict:
 def tune_batch(run) -> dict:
     """Picks the batched aligner's waves per CU with `run()` (one batch
     returning its work list: kernel microseconds per window level at [2:6]).
-    The 64-diagonal level's time depends only on its own waves and the wider
+    The first level's time depends only on its own waves and the wider
     levels' only on theirs (the tasks each level re-runs do not depend on the
     launch shape), so one run per candidate pair scores both."""
     base = current()

@@ -1,0 +1,74 @@
+"""The packed aligner (two alignments per wave, marvel_amd/csrc/la_pack.hpp)
+at the sizes where its paths change, against the oracle: batches that leave
+the upper halves idle and batches that use them, bands that stay within a
+half's 30 diagonals, that outgrow them for a while, and that outgrow the 128
+diagonals of the first wide window; trace spacings below and above the snake
+step, whose trace-point numbers wrap at 256; and initial bands of several
+diagonals up to and beyond a half."""
+
+import numpy as np
+import pytest
+
+import la_golden
+import oracle_lib
+from marvel_amd import latasks
+from marvel_amd.align import la_batch
+from marvel_amd.lib import MiTuning, lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ts):
+    want, st = oracle_lib.run_tasks(ts)
+    got, status = la_batch(ts)
+    keep = [i for i in range(ts.n) if st[i] == 0]
+    bad = la_golden.diff([got[i] for i in keep], [want[i] for i in keep], status[keep])
+    assert not bad, "\n".join(bad)
+    assert all(status[i] == 3 for i in range(ts.n) if st[i] != 0)
+    return len(keep)
+
+
+@pytest.fixture
+def few_waves():
+    """1,024 waves on 256 CUs: batches beyond that use both halves of a wave."""
+    import ctypes as C
+    t = MiTuning(0, 0, 0, 4, 0)
+    assert lib.mi_set_tuning(C.byref(t)) == 0
+    yield
+    lib.mi_set_tuning(None)
+
+
+@pytest.mark.parametrize("offmax", [0, 15, 40, 200])
+@pytest.mark.parametrize("tspace", [7, 100, 250])
+def test_bands_and_trace_spacings(tspace, offmax):
+    ts = latasks.make_tasks(48, 900 + offmax + tspace, lmin=300, lmax=4000, emin=0.02, emax=0.25, offmax=offmax,
+                            tspace=tspace)
+    print(f"[pack] tspace={tspace} offmax={offmax} n={ts.n}", flush=True)
+    assert _check(ts) >= 40
+
+
+@pytest.mark.parametrize("n", [1, 2, 1024, 1025, 2600])
+def test_one_and_two_alignments_per_wave(n, few_waves):
+    ts = latasks.make_tasks(n, 77 + n, lmin=200, lmax=700, emin=0.05, emax=0.25, offmax=30)
+    print(f"[pack] n={n}", flush=True)
+    _check(ts)
+
+
+@pytest.mark.parametrize("width", [2, 29, 30, 31, 90, 200])
+def test_initial_bands(width):
+    """Local_Alignment started on `width` diagonals around the seed's."""
+    ts = latasks.make_tasks(12, 300 + width, lmin=1500, lmax=3000, emin=0.05, emax=0.15, offmax=0)
+    par = ts.par.copy()
+    keep = []
+    for i in range(ts.n):
+        low = int(par[i, 3]) - width // 2
+        hgh = low + width - 1
+        alen, blen, anti = int(par[i, 0]), int(par[i, 1]), int(par[i, 5])
+        # every start point inside both reads
+        if all(0 <= (anti - k) // 2 <= blen and 0 <= (anti - k) // 2 + k <= alen for k in (low, hgh)):
+            par[i, 3], par[i, 4] = low, hgh
+            keep.append(i)
+    assert len(keep) >= 4
+    reads = [r for i in keep for r in (ts.reads[2 * i], ts.reads[2 * i + 1])]
+    print(f"[pack] width={width} n={len(keep)}", flush=True)
+    _check(latasks.TaskSet(ts.ave_corr, ts.tspace, ts.freq, reads, par[np.array(keep)]))

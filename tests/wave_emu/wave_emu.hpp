@@ -140,3 +140,11 @@ inline int __ffsll(long long x) { return __builtin_ffsll(x); }
 inline int __clzll(long long x) { return x ? __builtin_clzll((unsigned long long)x) : 64; }
 using std::max;
 using std::min;
+inline int __builtin_amdgcn_ds_bpermute(int addr, int v) { return emu::xchg(v, (addr >> 2) & 63); }
+inline unsigned __builtin_bitreverse32(unsigned x)
+{
+    unsigned r = 0;
+    for (int i = 0; i < 32; i++) r |= ((x >> i) & 1u) << (31 - i);
+    return r;
+}
+inline int __popc(unsigned x) { return __builtin_popcount(x); }
