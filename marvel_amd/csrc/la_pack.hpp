@@ -234,9 +234,17 @@ __device__ __forceinline__ void pack_tables(PackLds& L, const DevSpec& sp)
         L.w_match = all / 15;
         L.w_all = (all - none) / 15;
     }
+    // both halves idle: the loop reads every field of a slot, also of one that never gets an alignment
+    int* z = (int*)L.slot;
+    for (int i = lane; i < (int)(sizeof(L.slot) / sizeof(int)); i += 64) z[i] = 0;
+    z = (int*)L.band;
+    for (int i = lane; i < (int)(sizeof(L.band) / sizeof(int)); i += 64) z[i] = 0;
+    wave_sync();
     if (lane < 2) {
         L.slot[lane].phase = PH_IDLE;
-        L.slot[lane].running = 0;
+        L.slot[lane].a = 1;
+        L.slot[lane].amin = kFar;
+        L.slot[lane].bmax = -kFar;
     }
     wave_sync();
 }
