@@ -269,10 +269,10 @@ int mi_device_memset(void *p, int value, long long bytes);
 
 /* Launch shapes of the GPU kernels (no reference counterpart; results do
  * not depend on them): waves per CU of the report kernel's first window
- * (4..32, default 20; two pairs a wave) and of its 256-diagonal window (2..32,
+ * (4..32, default 24; two pairs a wave) and of its 256-diagonal window (2..32,
  * default 8), the pebble pool of the first window as a power of two (12..18,
  * default 15), waves per CU of the batched aligner's first window (4..32,
- * default 20) and of its 256-diagonal window (2..32, default 4).  A 0 field
+ * default 24) and of its 256-diagonal window (2..32, default 4).  A 0 field
  * keeps the default; NULL restores all defaults.
  * The tuner in marvel_amd/tune.py picks them from a calibration run. */
 typedef struct {

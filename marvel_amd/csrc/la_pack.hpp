@@ -37,15 +37,21 @@
 //   * What only changes at events lives in LDS, written by the lane that owns
 //     the event: the trim point, the best point's y, the boundary point.
 //
-// What bounds it: VALU issue -- 2.92e10 wave64 VALU instructions per report
-// launch on the 5 Mbp / 30x block, 47.6 ms of the 64 ms it takes at one per
-// SIMD every 4 cycles -- and waits on LDS and memory for the rest.  One
+// What bounds it, on a full GPU: VALU issue -- 2.59e10 wave64 VALU
+// instructions per report launch on the 5 Mbp / 30x block (190 per step of two
+// alignments), 42 ms of the 53 ms it takes at one per SIMD every 4 cycles; one
 // alignment per wave needed 5.2e10 and 96 ms (and 6.6 ms more for the pairs
-// wider than 64 diagonals, run again at 128).  Waves per SIMD: 4, 5 and 6 take
-// the same time there (211, 214, 213 ms a pass), 7 is slower (220 ms: its 72
-// registers spill in the loop); a repeat-rich block prefers few (227, 234,
-// 235, 262 ms), 400,000 tasks that start off their diagonal prefer many (69.2,
-// 65.2, 61.3, 60.7 ms), so 5.
+// wider than 64 diagonals, run again at 128).  So the sets of lanes are kept as
+// the compares' own masks (ballot, lane_in: an integer made of a condition and
+// compared again took 2 instructions more each, 64 ms a launch), products are
+// 24-bit, and the reads and the pool are addressed as HBM (a flat access also
+// holds up every wait for LDS).  Where few alignments are left (repeat-rich
+// blocks: one pair with 90 alignments one after another, 55 % of the CUs busy
+// over the launch) it is the latency of one wave's step, about 1.5 us.
+// Waves per SIMD: 4, 5, 6 and 7 take 190, 178, 175, 179 ms a pass on the 5 Mbp
+// block and 66, 74, 56, 56 ms on 400,000 tasks that start off their diagonal;
+// repeat-rich blocks prefer fewer (214, 212, 217, 218 ms).  7 spills in the
+// loop, so 6.
 //
 // Persistent kernels: `Job` (a few pointers, passed by value) hands out
 // alignments (next) and takes their results (done); PackSlot says what it
@@ -57,12 +63,13 @@
 namespace mi {
 
 constexpr int kHalfBand = 30;          // diagonals a half holds (lanes 1..30)
-constexpr int kNarrow = 24;            // a wide band this narrow returns to its half
+constexpr int kNarrow = 18;            // a wide band this narrow returns to its half
+constexpr int kOneChunk = 44;          // a wide band this narrow is kept in one 64-lane chunk, the others' steps are skipped
 constexpr int kSentV = -(1 << 30);     // V of a lane without a diagonal
 constexpr int kFar = 1 << 30;          // no border
 constexpr int kPebIdx = 0xffffff;      // pebble index in HA / HB; the top 8 bits: its trace point's number
 constexpr int kPoolMax = 1 << 24;
-constexpr int kPackWaves = 5;          // waves per SIMD of the kernels with the smallest wide window (see the note above)
+constexpr int kPackWaves = 6;          // waves per SIMD of the kernels with the smallest wide window (see the note above)
 constexpr int kSufBits = 10;           // columns per lookup of the suffix table
 
 // phases of a slot
@@ -84,15 +91,13 @@ struct PackSlot {
     int mind;            // reverse pass: the diagonal of the forward B chain's root
     int status;          // LA_* it ended with
     int used, dif;       // pebbles, waves
-    int best_y;
-    int tr_c, tr_y, tr_d, tr_ha, tr_hb;           // trim point
-    int mo_m, mo_c, mo_y, mo_d, mo_ha, mo_hb;     // boundary point (mo_m < 0: none)
     int fa, fb;          // forward trace lengths
     // the alignment's results
     long long cells, snake, steps, snake0;   // snake0: before the pass
     LaResult res;
     // a pass outside the loop's registers (see PackBand)
     int a, b, ktop, besta, lasta, navail, amin, bmax, running;
+    int prio;            // the wave's priority while this alignment runs (queue_priority)
 };
 
 // A half's diagonals outside the loop's registers: while the other half is
@@ -103,7 +108,16 @@ struct PackBand {
 };
 constexpr int kEnd = 1 << 16;
 
+// What the loop writes at events, at the front of LDS (small offsets).
+struct PackHot {
+    int tr_c, tr_y, tr_d, tr_ha, tr_hb;           // trim point
+    int best_y;                                   // y of the best antidiagonal's diagonal
+    int mo_m, mo_c, mo_y, mo_d, mo_ha, mo_hb;     // boundary point (mo_m < 0: none)
+    int pad[4];
+};
+
 struct PackLds {
+    PackHot hot[2];
     int16_t suf[1 << kSufBits];   // smallest suffix sum of 10 columns given by their mismatches
     int w_all, w_match;           // score of a column: w_match for a match, w_match - w_all for a mismatch
     DevSpec sp;
@@ -115,6 +129,8 @@ struct PackLds {
 // through the kernarg segment, so none of it is held across the loop.
 #ifndef MI_CPU_WAVE_EMU
 template <class T>
+using Glob = T __attribute__((address_space(1)));   // in HBM: pointers that come out of LDS would be flat otherwise
+template <class T>
 using KernArgs = const T __attribute__((address_space(4)));
 template <class T>
 __device__ __forceinline__ const T* kernarg_ptr()
@@ -124,10 +140,34 @@ __device__ __forceinline__ const T* kernarg_ptr()
 #else
 // the CPU wave emulator (tests/wave_emu) hands the launch's arguments over
 template <class T>
+using Glob = T;
+template <class T>
 using KernArgs = const T;
 template <class T>
 inline const T* kernarg_ptr() { return (const T*)emu::kernarg(); }
 #endif
+
+// the lanes where p holds: the compare's own mask (HIP's __ballot makes an integer of p and compares it again)
+__device__ __forceinline__ unsigned long long ballot(bool p)
+{
+#ifndef MI_CPU_WAVE_EMU
+    return __builtin_amdgcn_ballot_w64(p);
+#else
+    return __ballot(p);
+#endif
+}
+__device__ __forceinline__ bool any_lane(bool p) { return ballot(p) != 0; }
+// whether this lane is one of m's: the mask itself as the condition
+__device__ __forceinline__ bool lane_in(unsigned long long m)
+{
+#ifndef MI_CPU_WAVE_EMU
+    return __builtin_amdgcn_inverse_ballot_w64(m);
+#else
+    return (m >> __lane_id()) & 1;
+#endif
+}
+typedef int Int4 __attribute__((vector_size(16)));   // a pebble as it is stored
+static_assert(sizeof(Peb) == 16, "a pebble is stored as one vector");
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 template <class T>
@@ -147,6 +187,15 @@ __device__ __forceinline__ KernArgs<T>* kern_args(const T* p)
 {
     return (KernArgs<T>*)uni(p);
 }
+// product of two factors below 2^23 (full rate; the 32-bit multiply takes four times as long)
+__device__ __forceinline__ int mul24(int x, int y)
+{
+#ifndef MI_CPU_WAVE_EMU
+    return __mul24(x, y);
+#else
+    return x * y;
+#endif
+}
 // value of lane `src`
 __device__ __forceinline__ int bperm(int v, int src) { return __builtin_amdgcn_ds_bpermute(src << 2, v); }
 __device__ __forceinline__ uint64_t bperm64(uint64_t v, int src)
@@ -158,12 +207,30 @@ __device__ __forceinline__ int hsel(int hm, int lo, int hi)
 {
     return (int)((unsigned)lo + ((unsigned)hm & ((unsigned)hi - (unsigned)lo)));
 }
+// Wave priority (0..3) by the place in the queue: the queues hold the longest
+// alignments first, and a launch ends when the longest chain of waves does,
+// so the waves that hold it issue before the others of their SIMD.
+// (A 4 Mbp block 13.3 -> 11.7 ms a pass, 400,000 tasks 50.2 -> 46.7 ms; blocks
+// whose heavy pairs their seeds do not tell, 246.9 and 249.6 ms.)
+__device__ __forceinline__ int queue_priority(int t, int n)
+{
+    return t < n / 256 ? 3 : t < n / 32 ? 2 : t < n / 8 ? 1 : 0;
+}
+__device__ __forceinline__ void set_priority(int p)
+{
+#ifndef MI_CPU_WAVE_EMU
+    if (p == 3) __builtin_amdgcn_s_setprio(3);
+    else if (p == 2) __builtin_amdgcn_s_setprio(2);
+    else if (p == 1) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+#endif
+}
 __device__ __forceinline__ uint32_t hmask(int hm, unsigned long long m)
 {
     return (uint32_t)hsel(hm, (int)(uint32_t)m, (int)(uint32_t)(m >> 32));
 }
-__device__ __forceinline__ int top_bit(uint32_t m) { return 31 - __builtin_clz(m); }   // m != 0
-__device__ __forceinline__ int low_bit(uint32_t m) { return __builtin_ctz(m); }        // m != 0
+__device__ __forceinline__ int top_bit(uint32_t m) { return 31 - __builtin_clz(m | 1u); }
+__device__ __forceinline__ int low_bit(uint32_t m) { return __builtin_ctz(m | 0x80000000u); }
 
 // inclusive prefix maximum over the lanes of each half / of the wave
 template <int CTRL, int ROWS = 0xF>
@@ -182,23 +249,46 @@ __device__ __forceinline__ int prefix_max(int x)
     if constexpr (WAVE) x = dpp_max<0x143, 0xC>(x);   // row_bcast:31 into rows 2, 3
     return x;
 }
+// value of lane L - 1 / L + 1; lanes 0 / 63: anything / the sentinel
+__device__ __forceinline__ int dpp_shr1(int v) { return __builtin_amdgcn_mov_dpp(v, 0x138, 0xF, 0xF, true); }
+__device__ __forceinline__ int dpp_shl1(int v) { return __builtin_amdgcn_mov_dpp(v, 0x130, 0xF, 0xF, true); }
 __device__ __forceinline__ int from_below(int v) { return __builtin_amdgcn_update_dpp(kSentV, v, 0x138, 0xF, 0xF, false); }
 __device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_update_dpp(kSentV, v, 0x130, 0xF, 0xF, false); }
 
 // Matching columns from (x, y) on in the pass's direction, at most lim (m: 0
-// forward, -1 reverse; x and y in the pass's coordinates).  16 bases a step.
-__device__ __forceinline__ int snake_len(const uint32_t* A, const uint32_t* B, int m, int x, int y, int lim)
+// forward, -1 reverse; x and y in the pass's coordinates), on the lanes where
+// `in` holds; every lane takes part.  32 bases a step: a second step is a
+// round trip to memory for the whole wave, and with 16 bases one of its lanes
+// asked for it in 9 of 10 steps at 16 % pair error (in 1 of 8 at 28 %).
+// (repeat-rich block 246.9 -> 242.3 ms a pass, long reads 235.1 -> 230.4 ms,
+// 64 tasks 3.27 -> 3.18 ms; the 28 % block 176.5 and 178.1 ms.)
+typedef Glob<const uint32_t> SeqWord;
+// the 32-base windows at x and y compared: bit pair i differs where base i does
+__device__ __forceinline__ uint64_t seq_diff(SeqWord* A, SeqWord* B, int m, int x, int y)
+{
+    const int off = m & -31;
+    const int p = (x ^ m) + off, q = (y ^ m) + off;   // reverse: the 32 bases before x
+    SeqWord* a = A + (p >> 4);
+    SeqWord* b = B + (q >> 4);
+    const uint32_t a0 = a[0], a1 = a[1], a2 = a[2], b0 = b[0], b1 = b[1], b2 = b[2];
+    const uint32_t lo = __builtin_amdgcn_alignbit(a1, a0, (uint32_t)(2 * p)) ^
+                        __builtin_amdgcn_alignbit(b1, b0, (uint32_t)(2 * q));
+    const uint32_t hi = __builtin_amdgcn_alignbit(a2, a1, (uint32_t)(2 * p)) ^
+                        __builtin_amdgcn_alignbit(b2, b1, (uint32_t)(2 * q));
+    const uint32_t d0 = m ? __builtin_bitreverse32(hi) : lo, d1 = m ? __builtin_bitreverse32(lo) : hi;
+    return ((uint64_t)d1 << 32) | d0;
+}
+__device__ __forceinline__ int same_bases(uint64_t d) { return (d ? __builtin_ctzll(d) : 64) >> 1; }
+__device__ __forceinline__ int snake_len(SeqWord* A, SeqWord* B, int m, int x, int y, int lim, bool in)
 {
     int s = 0;
-    const int off = m & -15;
-    while (s < lim) {
-        const uint32_t d = win16(A, ((x + s) ^ m) + off) ^ win16(B, ((y + s) ^ m) + off);
-        const uint32_t r = m ? __builtin_bitreverse32(d) : d;
-        if (r) {
-            s += __builtin_ctz(r) >> 1;
-            break;
-        }
-        s += 16;
+    if (in) s = same_bases(seq_diff(A, B, m, x, y));
+    unsigned long long go = ballot(s == 32) & ballot(lim > 32);
+    while (go) {
+        int n = 0;
+        if (lane_in(go)) n = same_bases(seq_diff(A, B, m, x + s, y + s));
+        s += n;
+        go = ballot(n == 32) & ballot(s < lim);
     }
     return min(s, lim);
 }
@@ -214,14 +304,15 @@ __device__ __forceinline__ void add_columns(uint64_t& N, int& m, int s)
 }
 constexpr uint64_t kColsInit = (1ull << 63) | 4;   // 60 matches
 
-// every suffix of the last 30 columns has a score >= 0 (TABLE and SCORE of dalign/align.c:884-896)
-__device__ __forceinline__ bool suffix_positive(const PackLds& L, uint64_t N)
+// the smallest score of a suffix of the last 30 columns; >= 0: the path may be trimmed here (TABLE and SCORE of
+// dalign/align.c:884-896)
+__device__ __forceinline__ int min_suffix(const PackLds& L, int w_match, int w_all, uint64_t N)
 {
     const uint32_t z = (uint32_t)(N >> 3) & 0x3fffffffu;
-    const int s1 = 10 * L.w_match - __popc(z & 0x3ffu) * L.w_all;
-    const int s2 = 20 * L.w_match - __popc(z & 0xfffffu) * L.w_all;
+    const int s1 = 10 * w_match - mul24(__popc(z & 0x3ffu), w_all);
+    const int s2 = 20 * w_match - mul24(__popc(z & 0xfffffu), w_all);
     const int q0 = L.suf[z & 0x3ffu], q1 = L.suf[(z >> 10) & 0x3ffu] + s1, q2 = L.suf[z >> 20] + s2;
-    return min(q0, min(q1, q2)) >= 0;
+    return min(q0, min(q1, q2));
 }
 
 __device__ __forceinline__ void pack_tables(PackLds& L, const DevSpec& sp)
@@ -239,6 +330,8 @@ __device__ __forceinline__ void pack_tables(PackLds& L, const DevSpec& sp)
     for (int i = lane; i < (int)(sizeof(L.slot) / sizeof(int)); i += 64) z[i] = 0;
     z = (int*)L.band;
     for (int i = lane; i < (int)(sizeof(L.band) / sizeof(int)); i += 64) z[i] = 0;
+    z = (int*)L.hot;
+    for (int i = lane; i < (int)(sizeof(L.hot) / sizeof(int)); i += 64) z[i] = 0;
     wave_sync();
     if (lane < 2) {
         L.slot[lane].phase = PH_IDLE;
@@ -263,6 +356,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
     constexpr int W = 64 * NCH;
     const int lane = __lane_id();
     PackSlot& S = L->slot[h];
+    PackHot& H = L->hot[h];
     PackBand& D = L->band[h];
     const int TS = uni(L->sp.tspace), ave = uni(L->sp.ave_path);
     const int alen = uni(S.alen), blen = uni(S.blen);
@@ -270,9 +364,10 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
     const int boff = uni(S.comp) ? blen % TS : 0;
     const int offB = (boff ^ m) - m;
     const int limA = alen & ~m, limB = blen & ~m;
-    const uint32_t* A = (const uint32_t*)uni(S.A);
-    const uint32_t* B = (const uint32_t*)uni(S.B);
-    Peb* pool = uni(S.pool);
+    SeqWord* A = (SeqWord*)uni(S.A);
+    SeqWord* B = (SeqWord*)uni(S.B);
+    Glob<Int4>* pool = (Glob<Int4>*)uni(S.pool);
+    const int w_match = uni(L->w_match), w_all = uni(L->w_all);
     const int cap = uni(S.pool_cap);
     int a = uni(S.a), b = uni(S.b), kt = uni(S.ktop), besta = uni(S.besta), lasta = uni(S.lasta), dif = uni(S.dif);
     int navail = uni(S.navail), amin = uni(S.amin), bmax = uni(S.bmax);
@@ -301,38 +396,43 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
             M[j] = HA[j] = HB[j] = tA[j] = tB[j] = y[j] = 0;
             N[j] = kColsInit;
             end[j] = false;
-            if (i < a || i > b || status != LA_OK) continue;
-            y[j] = (mida - k) >> 1;
-            const int x = y[j] + k;
-            const bool bad = y[j] < 0 || y[j] > blen || x < 0 || x > alen;
-            undef |= bad;
-            tA[j] = x / TS + 1;
-            tB[j] = (y[j] + (TS - boff)) / TS;
-            HA[j] = 2 * (i - a);
-            HB[j] = HA[j] + 1;
-            pool[HA[j]] = Peb{-1, k, 0, (tA[j] - 1) * TS};
-            pool[HB[j]] = Peb{-1, k, 0, (tB[j] - 1) * TS + boff};
-            HA[j] |= (int)((unsigned)(tA[j] - 1) << 24);
-            HB[j] |= (int)((unsigned)(tB[j] - 1) << 24);
-            M[j] = kPathLen;
-            if (i == a) {
-                S.best_y = S.tr_y = y[j];
-                S.tr_c = mida;
-                S.tr_d = 0;
-                S.tr_ha = 0;
-                S.tr_hb = 1;
-                S.mo_m = -1;
+            const bool in = i >= a && i <= b && status == LA_OK;
+            int lim = 0;
+            if (in) {
+                y[j] = (mida - k) >> 1;
+                const int x = y[j] + k;
+                const bool bad = y[j] < 0 || y[j] > blen || x < 0 || x > alen;
+                undef |= bad;
+                tA[j] = x / TS + 1;
+                tB[j] = (y[j] + (TS - boff)) / TS;
+                HA[j] = 2 * (i - a);
+                HB[j] = HA[j] + 1;
+                pool[HA[j]] = Int4{-1, k, 0, (tA[j] - 1) * TS};
+                pool[HB[j]] = Int4{-1, k, 0, (tB[j] - 1) * TS + boff};
+                HA[j] |= (int)((unsigned)(tA[j] - 1) << 24);
+                HB[j] |= (int)((unsigned)(tB[j] - 1) << 24);
+                M[j] = kPathLen;
+                if (i == a) {
+                    H.best_y = H.tr_y = y[j];
+                    H.tr_c = mida;
+                    H.tr_d = 0;
+                    H.tr_ha = 0;
+                    H.tr_hb = 1;
+                    H.mo_m = -1;
+                }
+                lim = bad ? 0 : min(alen - x, blen - y[j]);
             }
-            const int lim = bad ? 0 : min(alen - x, blen - y[j]);
-            const int s = snake_len(A, B, 0, x, y[j], lim);
-            end[j] = s == lim;
-            snake += s + 1;
-            y[j] += s;
-            V[j] = 2 * y[j] + k;
+            const int s = snake_len(A, B, 0, y[j] + k, y[j], lim, lim > 0);
+            if (in) {
+                end[j] = s == lim;
+                snake += s + 1;
+                y[j] += s;
+                V[j] = 2 * y[j] + k;
+            }
         }
-        if (status == LA_OK && __any(undef)) status = LA_UNDEF;
+        if (status == LA_OK && any_lane(undef)) status = LA_UNDEF;
     } else {
-        const int wd = b - a + 1, a1 = (W - wd) / 2, d = a1 - a;
+        const int wd = b - a + 1, d = (wd <= kOneChunk ? 64 - wd : W - wd) / 2 - a;
 #pragma unroll
         for (int j = 0; j < NCH; j++) {
             const int i = 64 * j + lane - d;   // lane in the half
@@ -361,13 +461,13 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
             // ---- the next wave: band one wider on each side (dalign/align.c:645-743)
             const bool ea = a - 1 >= amin, eb = b + 1 <= bmax;
             int na = ea ? a - 1 : a, nb = eb ? b + 1 : b;
-            if (na < 0 || nb >= W) {
-                const int wd = nb - na + 1;
+            const int wd = nb - na + 1;
+            if (na < 0 || nb >= W || (NCH > 1 && wd <= kOneChunk && (na >> 6) != (nb >> 6))) {
                 if (wd > W) {
                     status = LA_WIDE;
                     break;
                 }
-                const int d = na - (W - wd) / 2;   // index i takes index i + d
+                const int d = na - (wd <= kOneChunk ? 64 - wd : W - wd) / 2;   // index i takes index i + d
                 int v2[NCH], m2[NCH], ha2[NCH], hb2[NCH], ta2[NCH], tb2[NCH];
                 uint64_t n2[NCH];
 #pragma unroll
@@ -512,20 +612,20 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 const bool in = i >= a && i <= b;
                 const int mx = max(am[j], ap[j]);
                 int c = V[j] < mx ? mx + 1 : V[j] + 2;
+                if (in) y[j] = (c - k) >> 1;
+                const int x = y[j] + k, lim = in ? min(limA - x, limB - y[j]) : 0;
+                undef |= lim < 0;
+                const int s = max(snake_len(A, B, m, x, y[j], lim, lim > 0), 0);
                 V[j] = kSentV;
                 if (in) {
-                    y[j] = (c - k) >> 1;
-                    const int x = y[j] + k, lim = min(limA - x, limB - y[j]);
-                    if (lim < 0) undef = true;
-                    const int s = snake_len(A, B, m, x, y[j], lim);
                     end[j] = s == lim;
-                    snake += max(s, 0) + 1;
-                    add_columns(N[j], M[j], max(s, 0));
+                    snake += s + 1;
+                    add_columns(N[j], M[j], s);
                     y[j] += s;
                     V[j] = 2 * y[j] + k;
                 }
             }
-            if (__any(undef)) {
+            if (any_lane(undef)) {
                 status = LA_UNDEF;
                 break;
             }
@@ -534,7 +634,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 bool e = false;
 #pragma unroll
                 for (int j = 0; j < NCH; j++) e |= end[j];
-                if (!__any(e)) {
+                if (!any_lane(e)) {
                     const int d = a - (1 + (kHalfBand - (b - a + 1)) / 2);
 #pragma unroll
                     for (int j = 0; j < NCH; j++) {
@@ -575,18 +675,18 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
             for (int j = 0; j < NCH; j++) {
                 const int i = 64 * j + lane;
                 const bool in = i >= a && i <= b;
-                wA[j] = in && y[j] + kt - i >= tA[j] * TS;
-                wB[j] = in && y[j] >= tB[j] * TS + offB;
+                wA[j] = in && y[j] + kt - i >= mul24(tA[j], TS);
+                wB[j] = in && y[j] >= mul24(tB[j], TS) + offB;
                 any |= wA[j] | wB[j];
             }
-            if (!__any(any)) break;
+            if (!any_lane(any)) break;
 #pragma unroll
             for (int j = 0; j < NCH; j++) {
                 if (!live(j)) continue;
                 const int k = kt - (64 * j + lane);
                 const bool pA = wA[j] && (dif == 0 || (int)(((unsigned)tA[j] << 24) - ((unsigned)HA[j] & ~(unsigned)kPebIdx)) > 0);
                 const bool pB = wB[j] && (dif == 0 || (int)(((unsigned)tB[j] << 24) - ((unsigned)HB[j] & ~(unsigned)kPebIdx)) > 0);
-                const unsigned long long ba = __ballot(pA), bb = __ballot(pB);
+                const unsigned long long ba = ballot(pA), bb = ballot(pB);
                 const int ca = __popcll(ba), cb = __popcll(bb);
                 if (navail + ca + cb > cap) {
                     full = true;
@@ -594,12 +694,12 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 }
                 if (pA) {
                     const int q = navail + prefix_rank(ba);
-                    pool[q] = Peb{HA[j] & kPebIdx, (k ^ m) - m, dif, ((tA[j] * TS) ^ m) - m};
+                    pool[q] = Int4{HA[j] & kPebIdx, (k ^ m) - m, dif, ((tA[j] * TS) ^ m) - m};
                     HA[j] = q | (int)((unsigned)tA[j] << 24);
                 }
                 if (pB) {
                     const int q = navail + ca + prefix_rank(bb);
-                    pool[q] = Peb{HB[j] & kPebIdx, (k ^ m) - m, dif, ((tB[j] * TS + offB) ^ m) - m};
+                    pool[q] = Int4{HB[j] & kPebIdx, (k ^ m) - m, dif, ((tB[j] * TS + offB) ^ m) - m};
                     HB[j] = q | (int)((unsigned)tB[j] << 24);
                 }
                 navail += ca + cb;
@@ -622,18 +722,18 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 const int e = __builtin_amdgcn_update_dpp(carry, incl, 0x138, 0xF, 0xF, false);
                 const bool rec = V[j] > max(e, carry);
                 carry = max(carry, rdl(incl, 63));
-                if (rec && V[j] == carry) S.best_y = y[j];
+                if (rec && V[j] == carry) H.best_y = y[j];
                 const bool good = rec && (dif == 0 || M[j] >= ave);
-                const unsigned long long bm = __ballot(good);
+                const unsigned long long bm = ballot(good);
                 if (bm) {
                     lasta = rdl(V[j], highest_lane(bm));
-                    const unsigned long long bt = __ballot(good && (dif == 0 || suffix_positive(*L, N[j])));
+                    const unsigned long long bt = ballot(good && (dif == 0 || min_suffix(*L, w_match, w_all, N[j]) >= 0));
                     if (bt && lane == highest_lane(bt)) {
-                        S.tr_c = V[j];
-                        S.tr_y = y[j];
-                        S.tr_d = dif;
-                        S.tr_ha = HA[j] & kPebIdx;
-                        S.tr_hb = HB[j] & kPebIdx;
+                        H.tr_c = V[j];
+                        H.tr_y = y[j];
+                        H.tr_d = dif;
+                        H.tr_ha = HA[j] & kPebIdx;
+                        H.tr_hb = HB[j] & kPebIdx;
                     }
                 }
             }
@@ -648,15 +748,15 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
 #pragma unroll
             for (int j = 0; j < NCH; j++) {
                 if (!live(j)) continue;
-                const unsigned long long eb_ = __ballot(end[j] && y[j] == limB);
-                const unsigned long long ea_ = __ballot(end[j] && y[j] != limB);
+                const unsigned long long eb_ = ballot(end[j] && y[j] == limB);
+                const unsigned long long ea_ = ballot(end[j] && y[j] != limB);
                 if (ea_) la = 64 * j + highest_lane(ea_);
                 if (eb_) lb = min(lb, 64 * j + lowest_lane(eb_));
                 any |= (ea_ | eb_) != 0;
             }
             if (any) {
                 wave_sync();
-                const int by = uni(S.best_y);
+                const int by = uni(H.best_y);
                 more = (by == limB || besta - by == limA) ? 0 : 1;
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
@@ -665,16 +765,16 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                     if (!hit) continue;
                     if (q == 0) a = at + 1;
                     else b = at - 1;
-                    const int mo = uni(S.mo_m);
+                    const int mo = uni(H.mo_m);
 #pragma unroll
                     for (int j = 0; j < NCH; j++)
                         if (64 * j + lane == at && mo <= M[j]) {
-                            S.mo_m = M[j];
-                            S.mo_c = V[j];
-                            S.mo_y = y[j];
-                            S.mo_d = dif;
-                            S.mo_ha = HA[j] & kPebIdx;
-                            S.mo_hb = HB[j] & kPebIdx;
+                            H.mo_m = M[j];
+                            H.mo_c = V[j];
+                            H.mo_y = y[j];
+                            H.mo_d = dif;
+                            H.mo_ha = HA[j] & kPebIdx;
+                            H.mo_hb = HB[j] & kPebIdx;
                         }
                     wave_sync();
                 }
@@ -687,7 +787,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
 #pragma unroll
             for (int j = 0; j < NCH; j++) {
                 const int i = 64 * j + lane;
-                const unsigned long long bk = __ballot(i >= a && i <= b && V[j] >= n);
+                const unsigned long long bk = ballot(i >= a && i <= b && V[j] >= n);
                 if (bk) {
                     na2 = min(na2, 64 * j + lowest_lane(bk));
                     nb2 = 64 * j + highest_lane(bk);
@@ -736,6 +836,7 @@ __device__ __noinline__ void pack_service(Job job, PackLds* L, int h)
 {
     const int lane = __lane_id();
     PackSlot& S = L->slot[h];
+    const PackHot& H = L->hot[h];
     const int TS = uni(L->sp.tspace);
     const int phase = uni(S.phase);
     if (phase != PH_IDLE) {
@@ -751,10 +852,10 @@ __device__ __noinline__ void pack_service(Job job, PackLds* L, int h)
         const int maxtp = uni(S.maxtp);
         uint16_t *atr = uni(S.atr), *btr = uni(S.btr);
         if (status == LA_OK) {
-            const bool mo = uni(S.mo_m) >= 0;
-            const int c = mo ? uni(S.mo_c) : uni(S.tr_c), yy = mo ? uni(S.mo_y) : uni(S.tr_y);
-            const int trimd = mo ? uni(S.mo_d) : uni(S.tr_d);
-            const int tha = mo ? uni(S.mo_ha) : uni(S.tr_ha), thb = mo ? uni(S.mo_hb) : uni(S.tr_hb);
+            const bool mo = uni(H.mo_m) >= 0;
+            const int c = mo ? uni(H.mo_c) : uni(H.tr_c), yy = mo ? uni(H.mo_y) : uni(H.tr_y);
+            const int trimd = mo ? uni(H.mo_d) : uni(H.tr_d);
+            const int tha = mo ? uni(H.mo_ha) : uni(H.tr_ha), thb = mo ? uni(H.mo_hb) : uni(H.tr_hb);
             const int trimx = rev ? yy - c : c - yy, trimy = rev ? -yy : yy;
             Peb* pool = uni(S.pool);
             const int pts_cap = uni(S.pts_cap);
@@ -850,6 +951,7 @@ static __device__ __noinline__ void pass_begin(PackLds* L, int h)
 {
     const int lane = __lane_id(), sl = lane & 31;
     PackSlot& S = L->slot[h];
+    PackHot& H = L->hot[h];
     PackBand& D = L->band[h];
     const int TS = uni(L->sp.tspace);
     const bool rev = uni(S.phase) == PH_REV;
@@ -864,58 +966,56 @@ static __device__ __noinline__ void pass_begin(PackLds* L, int h)
     if (2 * wd > cap || cap > kPoolMax) status = LA_POOL;
     else if (wd > kHalfBand) status = LA_GROW;
     bool bad = false;
-    int snake = 0;
-    if (status == LA_OK && lane < 32) {
-        int V = kSentV, M = 0, HA = 0, HB = 0, tA = 0, tB = 0;
-        if (sl >= a && sl <= b) {
-            Peb* pool = S.pool;
-            const int kr = (k ^ m) - m;
-            const int yr = (mida - kr) >> 1, xr = yr + kr;
-            bad = yr < 0 || yr > blen || xr < 0 || xr > alen;
-            int ma, mb;   // the roots' marks
-            if (!rev) {
-                const int na = xr / TS, nb = (yr + (TS - boff)) / TS - 1;
-                tA = na + 1;
-                tB = nb + 1;
-                ma = na * TS;
-                mb = nb * TS + boff;
-            } else {
-                tA = -((xr + TS - 1) / TS - 1);
-                tB = -((yr + (TS - boff) - 1) / TS - 1);
-                ma = xr;
-                mb = yr;
-            }
-            HA = 2 * (sl - a);
-            HB = HA + 1;
-            pool[HA] = Peb{-1, kr, 0, ma};
-            pool[HB] = Peb{-1, kr, 0, mb};
-            HA |= (int)((unsigned)(tA - 1) << 24);
-            HB |= (int)((unsigned)(tB - 1) << 24);
-            const int y = (yr ^ m) - m;
-            if (sl == a) {
-                S.best_y = S.tr_y = y;
-                S.tr_c = rev ? -mida : mida;
-                S.tr_d = 0;
-                S.tr_ha = 0;
-                S.tr_hb = 1;
-                S.mo_m = -1;
-            }
-            const int x = y + k, lim = bad ? 0 : min((rev ? 0 : alen) - x, (rev ? 0 : blen) - y);
-            const int s = snake_len((const uint32_t*)S.A, (const uint32_t*)S.B, m, x, y, lim);
-            snake = s + 1;
-            // the columns of a first wave are matches only
-            M = kPathLen | (s == lim ? kEnd : 0);
-            V = 2 * (y + s) + k;
+    const bool in = status == LA_OK && lane >= a && lane <= b;
+    int HA = 0, HB = 0, tA = 0, tB = 0, y = 0, lim = 0;
+    if (in) {
+        Glob<Int4>* pool = (Glob<Int4>*)S.pool;
+        const int kr = (k ^ m) - m;
+        const int yr = (mida - kr) >> 1, xr = yr + kr;
+        bad = yr < 0 || yr > blen || xr < 0 || xr > alen;
+        int ma, mb;   // the roots' marks
+        if (!rev) {
+            const int na = xr / TS, nb = (yr + (TS - boff)) / TS - 1;
+            tA = na + 1;
+            tB = nb + 1;
+            ma = na * TS;
+            mb = nb * TS + boff;
+        } else {
+            tA = -((xr + TS - 1) / TS - 1);
+            tB = -((yr + (TS - boff) - 1) / TS - 1);
+            ma = xr;
+            mb = yr;
         }
-        D.V[sl] = V;
-        D.M[sl] = M;
+        HA = 2 * (sl - a);
+        HB = HA + 1;
+        pool[HA] = Int4{-1, kr, 0, ma};
+        pool[HB] = Int4{-1, kr, 0, mb};
+        HA |= (int)((unsigned)(tA - 1) << 24);
+        HB |= (int)((unsigned)(tB - 1) << 24);
+        y = (yr ^ m) - m;
+        if (sl == a) {
+            H.best_y = H.tr_y = y;
+            H.tr_c = rev ? -mida : mida;
+            H.tr_d = 0;
+            H.tr_ha = 0;
+            H.tr_hb = 1;
+            H.mo_m = -1;
+        }
+        lim = bad ? 0 : min((rev ? 0 : alen) - (y + k), (rev ? 0 : blen) - y);
+    }
+    int snake = snake_len((SeqWord*)uni(S.A), (SeqWord*)uni(S.B), m, y + k, y, lim, lim > 0);
+    if (lane < 32) {
+        // the columns of a first wave are matches only
+        D.V[sl] = in ? 2 * (y + snake) + k : kSentV;
+        D.M[sl] = kPathLen | (in && snake == lim ? kEnd : 0);
         D.HA[sl] = HA;
         D.HB[sl] = HB;
         D.tA[sl] = tA;
         D.tB[sl] = tB;
         D.N[sl] = kColsInit;
     }
-    if (__any(bad)) status = LA_UNDEF;
+    snake = in ? snake + 1 : 0;
+    if (any_lane(bad)) status = LA_UNDEF;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) snake += __shfl_xor(snake, o, 64);
     if (lane == 0) {
@@ -965,6 +1065,7 @@ __device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, c
                     S.b = 0;
                     S.amin = kFar;
                     S.bmax = -kFar;
+                    S.prio = 0;
                 }
                 wave_sync();
                 break;
@@ -973,6 +1074,7 @@ __device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, c
             go = uni(S.status) == LA_OK;
         }
     }
+    set_priority(max(uni(L->slot[0].prio), uni(L->slot[1].prio)));
 }
 
 // ---- the loop --------------------------------------------------------------------------
@@ -983,171 +1085,202 @@ __device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, c
 template <int NCH, class Job>
 __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const int* abort_flag)
 {
-    const int lane = __lane_id(), sl = lane & 31, hm = -(lane >> 5);
-    PackSlot& S = L.slot[lane >> 5];
-    PackBand& D = L.band[lane >> 5];
-    const int TS = uni(L.sp.tspace), ave = uni(L.sp.ave_path);
-
-    // per diagonal; V, M, N, HA, HB as the reference's V, M, T, HA, HB; tA / tB: the numbers of the next trace points
-    int V = kSentV, M = 0, HA = 0, HB = 0, tA = 0, tB = 0, y = 0;
+    typedef unsigned long long Lanes;   // a set of lanes
+    // What serving a half would have to keep is set again after it (see below).
+    int lane = 0, sl = 0, hm = 0, TS = 0, ave = 0, w_all = 0, w_match = 0;
+    PackSlot* S = nullptr;
+    PackHot* H = nullptr;
+    PackBand* D = nullptr;
+    // per diagonal; V, M, N, HA, HB as the reference's V, M, T, HA, HB; tA / tB: the numbers of the next trace
+    // points; rem: columns left to a read's end (0: the wave's snake ran into it)
+    int V = kSentV, M = 0, HA = 0, HB = 0, tA = 0, tB = 0, y = 0, rem = 1;
     uint64_t N = 0;
-    bool end = false;   // the wave's snake ran into the end of a read
     // per half (the same on its 32 lanes); an idle half has an empty band that no border lets grow
     int k = 0, a = 1, b = 0, besta = 0, lasta = 0, dif = 0, navail = 0, amin = kFar, bmax = -kFar;
     int limA = 0, limB = 0, m = 0, offB = 0, cap = 0;
-    const uint32_t *A = nullptr, *B = nullptr;
-    Peb* pool = nullptr;
+    SeqWord *A = nullptr, *B = nullptr;
+    Glob<Int4>* pool = nullptr;
     int ncell = 0, nsnake = 0;
-    unsigned stopped = second ? 3u : 1u;   // halves to serve (bit 0: lanes 0..31)
+    // wave-uniform
+    Lanes act = 0, fresh = 0;                // halves with a pass; of these, in wave 0
+    unsigned stopped = second ? 3u : 1u;     // halves to serve (bit 0: lanes 0..31)
+    unsigned tick = 0;
 
     for (;;) {
         if (stopped) {
             // Nothing stays in registers while the wave serves a half: the
-            // other one's pass goes through LDS, so the loop does not pay for
-            // the registers of what it calls.
-            if (!((stopped >> (lane >> 5)) & 1)) {
-                D.V[sl] = V;
-                D.M[sl] = M | (end ? kEnd : 0);
-                D.HA[sl] = HA;
-                D.HB[sl] = HB;
-                D.tA[sl] = tA;
-                D.tB[sl] = tB;
-                D.N[sl] = N;
+            // other one's pass goes through LDS and everything else is set
+            // again, so the loop does not pay for the registers of what it
+            // calls.
+            if (lane_in(act) && !((stopped >> (lane >> 5)) & 1)) {
+                D->V[sl] = V;
+                D->M[sl] = M | (rem == 0 ? kEnd : 0);
+                D->HA[sl] = HA;
+                D->HB[sl] = HB;
+                D->tA[sl] = tA;
+                D->tB[sl] = tB;
+                D->N[sl] = N;
                 if (sl == 0) {
-                    S.a = a;
-                    S.b = b;
-                    S.ktop = k;
-                    S.besta = besta;
-                    S.lasta = lasta;
-                    S.dif = dif;
-                    S.navail = navail;
-                    S.amin = amin;
-                    S.bmax = bmax;
+                    S->a = a;
+                    S->b = b;
+                    S->ktop = k;
+                    S->besta = besta;
+                    S->lasta = lasta;
+                    S->dif = dif;
+                    S->navail = navail;
+                    S->amin = amin;
+                    S->bmax = bmax;
+                }
+            }
+            if (tick) {   // (the first time there is nothing to hand over)
+#pragma unroll
+                for (int o = 16; o >= 1; o >>= 1) nsnake += __shfl_xor(nsnake, o, 64);
+                if (sl == 0) {
+                    S->cells += ncell;
+                    S->snake += nsnake;
                 }
             }
             wave_sync();
             pack_serve<NCH>(job, &L, stopped, abort_flag);
             stopped = 0;
-            const bool rev = S.phase == PH_REV;
+            lane = __lane_id();
+#ifndef MI_CPU_WAVE_EMU
+            asm volatile("" : "+v"(lane));   // computed here, not once before the loop
+#endif
+            sl = lane & 31;
+            hm = -(lane >> 5);
+            S = &L.slot[lane >> 5];
+            H = &L.hot[lane >> 5];
+            D = &L.band[lane >> 5];
+            TS = uni(L.sp.tspace);
+            ave = uni(L.sp.ave_path);
+            w_all = uni(L.w_all);
+            w_match = uni(L.w_match);
+            const bool rev = S->phase == PH_REV;
             m = rev ? -1 : 0;
-            limA = rev ? 0 : S.alen;
-            limB = rev ? 0 : S.blen;
-            const int boff = S.comp ? S.blen % TS : 0;
+            limA = rev ? 0 : S->alen;
+            limB = rev ? 0 : S->blen;
+            const int boff = S->comp ? S->blen % TS : 0;
             offB = rev ? -boff : boff;
-            A = (const uint32_t*)S.A;
-            B = (const uint32_t*)S.B;
-            pool = S.pool;
-            cap = S.pool_cap;
-            a = S.a;
-            b = S.b;
-            k = S.ktop - sl;
-            besta = S.besta;
-            lasta = S.lasta;
-            dif = S.dif;
-            navail = S.navail;
-            amin = S.amin;
-            bmax = S.bmax;
+            A = (SeqWord*)S->A;
+            B = (SeqWord*)S->B;
+            pool = (Glob<Int4>*)S->pool;
+            cap = S->pool_cap;
+            a = S->a;
+            b = S->b;
+            k = S->ktop - sl;
+            besta = S->besta;
+            lasta = S->lasta;
+            dif = S->dif;
+            navail = S->navail;
+            amin = S->amin;
+            bmax = S->bmax;
             const bool in = sl >= a && sl <= b;
-            V = in ? D.V[sl] : kSentV;
-            M = D.M[sl];
-            end = in && (M & kEnd) != 0;
+            V = in ? D->V[sl] : kSentV;
+            M = D->M[sl];
+            rem = in && (M & kEnd) ? 0 : 1;
             M &= kEnd - 1;
-            HA = D.HA[sl];
-            HB = D.HB[sl];
-            tA = D.tA[sl];
-            tB = D.tB[sl];
-            N = D.N[sl];
+            HA = D->HA[sl];
+            HB = D->HB[sl];
+            tA = D->tA[sl];
+            tB = D->tB[sl];
+            N = D->N[sl];
             y = (V - k) >> 1;
+            ncell = nsnake = 0;
+            act = ballot(S->phase != PH_IDLE);
+            if (!act) break;   // every half is idle
+            fresh = act & ballot(dif == 0);
             wave_sync();
         }
-        if (__ballot(a <= b) == 0) break;   // every half is idle
 
         // ---- trace-point pebbles: wave 0 pushes always, later waves when the
         // inherited pebble does not already sit on the trace point
         // (dalign/align.c:521-563, :826-878, :1258-1297, :1562-1612)
-        const bool in = sl >= a && sl <= b;
-        bool full = false;
-        for (;;) {
-            const bool wA = in && y + k >= tA * TS, wB = in && y >= tB * TS + offB;
-            if (!__any(wA | wB)) break;
-            const bool pA = wA && (dif == 0 || (int)(((unsigned)tA << 24) - ((unsigned)HA & ~(unsigned)kPebIdx)) > 0);
-            const bool pB = wB && (dif == 0 || (int)(((unsigned)tB << 24) - ((unsigned)HB & ~(unsigned)kPebIdx)) > 0);
-            const unsigned long long ba = __ballot(pA), bb = __ballot(pB);
-            const int al = __popcll(ba & 0xffffffffull), bl = __popcll(bb & 0xffffffffull);
-            const int ah = __popcll(ba >> 32), bh = __popcll(bb >> 32);
-            const int ca = hsel(hm, al, ah), cb = hsel(hm, bl, bh);
-            full |= navail + ca + cb > cap;
-            if (pA && !full) {
-                const int q = navail + prefix_rank(ba) - (hm & al);
-                pool[q] = Peb{HA & kPebIdx, (k ^ m) - m, dif, ((tA * TS) ^ m) - m};
-                HA = q | (int)((unsigned)tA << 24);
+        {
+            const int x = y + k;
+            int nA = mul24(tA, TS), nB = mul24(tB, TS) + offB;
+            const Lanes in = ballot(sl >= a) & ballot(sl <= b);
+            Lanes wA = in & ballot(x >= nA), wB = in & ballot(y >= nB);
+            while (wA | wB) {
+                const Lanes pA = wA & (fresh | ballot((int)(((unsigned)tA << 24) - ((unsigned)HA & ~(unsigned)kPebIdx)) > 0));
+                const Lanes pB = wB & (fresh | ballot((int)(((unsigned)tB << 24) - ((unsigned)HB & ~(unsigned)kPebIdx)) > 0));
+                const int al = __popcll(pA & 0xffffffffull), bl = __popcll(pB & 0xffffffffull);
+                const int ia = navail + prefix_rank(pA) - (hm & al);
+                navail += hsel(hm, al, __popcll(pA >> 32));
+                const int ib = navail + prefix_rank(pB) - (hm & bl);
+                navail += hsel(hm, bl, __popcll(pB >> 32));
+                const Lanes room = ballot(navail <= cap);   // (once there is none, the pass stops below)
+                const int kr = (k ^ m) - m;
+                if (lane_in(pA & room)) {
+                    pool[(unsigned)ia] = Int4{HA & kPebIdx, kr, dif, (nA ^ m) - m};
+                    HA = ia | (int)((unsigned)tA << 24);
+                }
+                if (lane_in(pB & room)) {
+                    pool[(unsigned)ib] = Int4{HB & kPebIdx, kr, dif, (nB ^ m) - m};
+                    HB = ib | (int)((unsigned)tB << 24);
+                }
+                tA += lane_in(wA) ? 1 : 0;
+                tB += lane_in(wB) ? 1 : 0;
+                nA = mul24(tA, TS);
+                nB = mul24(tB, TS) + offB;
+                wA &= ballot(x >= nA);
+                wB &= ballot(y >= nB);
             }
-            if (pB && !full) {
-                const int q = navail + ca + prefix_rank(bb) - (hm & bl);
-                pool[q] = Peb{HB & kPebIdx, (k ^ m) - m, dif, ((tB * TS + offB) ^ m) - m};
-                HB = q | (int)((unsigned)tB << 24);
-            }
-            navail += ca + cb;
-            if (wA) tA += 1;
-            if (wB) tB += 1;
         }
 
         // ---- records: strict improvements of besta in lane order
         {
             const int incl = prefix_max<false>(V);
-            int e = from_below(incl);
+            int e = dpp_shr1(incl);
             e = sl == 0 ? besta : max(e, besta);
-            const bool rec = V > e;
             besta = max(besta, bperm(incl, lane | 31));
-            if (rec && V == besta) S.best_y = y;
-            const bool good = rec && (dif == 0 || M >= ave);
-            const unsigned long long bm = __ballot(good);
-            if (bm) {
-                const uint32_t mm = hmask(hm, bm);
-                const int lv = bperm(V, (lane & 32) + (mm ? top_bit(mm) : 0));
-                if (mm) lasta = lv;
-                bool t = false;
-                if (good) t = dif == 0 || suffix_positive(L, N);
-                const uint32_t mt = hmask(hm, __ballot(t));
-                if ((mt >> sl) == 1u) {   // the last one in visiting order
-                    S.tr_c = V;
-                    S.tr_y = y;
-                    S.tr_d = dif;
-                    S.tr_ha = HA & kPebIdx;
-                    S.tr_hb = HB & kPebIdx;
+            const Lanes rec = ballot(V > e);
+            if (lane_in(rec & ballot(V == besta))) H->best_y = y;
+            const Lanes good = rec & (fresh | ballot(M >= ave));
+            if (good) {
+                const uint32_t mm = hmask(hm, good);
+                const int lv = bperm(V, (lane & 32) + top_bit(mm));
+                lasta = mm ? lv : lasta;
+                const Lanes trim = good & (fresh | ballot(min_suffix(L, w_match, w_all, N) >= 0));
+                if ((hmask(hm, trim) >> sl) == 1u) {   // the last one in visiting order
+                    H->tr_c = V;
+                    H->tr_y = y;
+                    H->tr_d = dif;
+                    H->tr_ha = HA & kPebIdx;
+                    H->tr_hb = HB & kPebIdx;
                 }
             }
         }
-        if (in) ncell += 1;
+        ncell += b - a + 1;
 
         // ---- clips at the read ends (dalign/align.c:589-625, :912-944, :1327-1361, :1650-1686)
-        bool more = true;
-        if (__any(end)) {
+        Lanes over = 0;   // halves whose best path reached a read's end
+        const Lanes end = ballot(rem == 0);
+        if (end) {
             wave_sync();
-            const uint32_t mB = hmask(hm, __ballot(end && y == limB)), mA = hmask(hm, __ballot(end && y != limB));
-            if (mA | mB) {
-                const int by = S.best_y;
-                more = !(by == limB || besta - by == limA);
-            }
+            const Lanes eB = end & ballot(y == limB);
+            const uint32_t mB = hmask(hm, eB), mA = hmask(hm, end & ~eB);
+            const int by = H->best_y;
+            over = ballot((mA | mB) != 0) & (ballot(by == limB) | ballot(besta - by == limA));
             const int la = mA ? top_bit(mA) : -1, lb = mB ? low_bit(mB) : 32;
             const bool hitA = mA && la >= a;
-            if (hitA && sl == la && S.mo_m <= M) {
-                S.mo_m = M;
-                S.mo_c = V;
-                S.mo_y = y;
-                S.mo_d = dif;
-                S.mo_ha = HA & kPebIdx;
-                S.mo_hb = HB & kPebIdx;
+            if (hitA && sl == la && H->mo_m <= M) {
+                H->mo_m = M;
+                H->mo_c = V;
+                H->mo_y = y;
+                H->mo_d = dif;
+                H->mo_ha = HA & kPebIdx;
+                H->mo_hb = HB & kPebIdx;
             }
             wave_sync();
             const bool hitB = mB && lb <= b;
-            if (hitB && sl == lb && S.mo_m <= M) {
-                S.mo_m = M;
-                S.mo_c = V;
-                S.mo_y = y;
-                S.mo_d = dif;
-                S.mo_ha = HA & kPebIdx;
-                S.mo_hb = HB & kPebIdx;
+            if (hitB && sl == lb && H->mo_m <= M) {
+                H->mo_m = M;
+                H->mo_c = V;
+                H->mo_y = y;
+                H->mo_d = dif;
+                H->mo_ha = HA & kPebIdx;
+                H->mo_hb = HB & kPebIdx;
             }
             wave_sync();
             if (hitA) a = la + 1;
@@ -1156,78 +1289,66 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
         }
 
         // ---- WAVE_LAG trim of the band's ends (dalign/align.c:946-955, :1688-1697)
-        const uint32_t mk = hmask(hm, __ballot(V >= (dif > 0 ? besta - kWaveLag : kSentV + 1)));
-        if (mk) {
-            a = low_bit(mk);
-            b = top_bit(mk);
-        } else {
-            a = 1;
-            b = 0;
-        }
-        if (sl < a || sl > b) V = kSentV;
+        int lag = besta - kWaveLag;
+        if (fresh) lag = lane_in(fresh) ? kSentV + 1 : lag;
+        const uint32_t mk = hmask(hm, ballot(V >= lag));
+        a = low_bit(mk);    // (an empty band: 31 .. 0)
+        b = top_bit(mk);
+        V = lane_in(ballot(sl >= a) & ballot(sl <= b)) ? V : kSentV;
 
         // ---- go on?  Then the band grows by one diagonal on each side (dalign/align.c:645-743)
-        const bool act = amin != kFar;   // the half has a pass
-        int st = -1;
-        if (!(more && lasta >= besta - kTrimMLag)) st = LA_OK;
-        else if (mk == 0) st = LA_UNDEF;   // empty band with the loop still running
-        if (full) st = LA_POOL;
-        const bool ea = a - 1 >= amin, eb = b + 1 <= bmax;
-        int na = ea ? a - 1 : a, nb = eb ? b + 1 : b;
-        if (st < 0 && nb - na + 1 > kHalfBand) st = LA_GROW;
-        if ((dif & 255) == 255) {
-            const int ab = __atomic_load_n(abort_flag, __ATOMIC_RELAXED);
-            if (st < 0 && ab) st = LA_ABORT;
-            if (st < 0 && dif > 2 * (S.alen + S.blen) + 1024) st = LA_UNDEF;
+        const Lanes ea = ballot(a > amin), eb = ballot(b < bmax);
+        int na = a - (lane_in(ea) ? 1 : 0), nb = b + (lane_in(eb) ? 1 : 0);
+        const Lanes run = ballot(lasta >= besta - kTrimMLag) & ~over;
+        Lanes stop = act & (~run | ballot(mk == 0) | ballot(nb - na >= kHalfBand) | ballot(navail > cap));
+        Lanes aborted = 0;
+        if ((++tick & 255u) == 0) {
+            if (uni(__atomic_load_n(abort_flag, __ATOMIC_RELAXED))) aborted = ~0ull;
+            stop |= act & (aborted | ballot(dif > 2 * (S->alen + S->blen) + 1024));
         }
-        const unsigned long long bs = __ballot(act && st >= 0);
-        if (bs) {
-            if (act && st == LA_GROW) {
-                D.V[sl] = V;
-                D.M[sl] = M;
-                D.HA[sl] = HA;
-                D.HB[sl] = HB;
-                D.tA[sl] = tA;
-                D.tB[sl] = tB;
-                D.N[sl] = N;
-            }
-            int tc = ncell, ts = nsnake;
-#pragma unroll
-            for (int o = 16; o >= 1; o >>= 1) {
-                tc += __shfl_xor(tc, o, 64);
-                ts += __shfl_xor(ts, o, 64);
-            }
-            if (sl == 0) {
-                S.cells += tc;
-                S.snake += ts;
-            }
-            ncell = nsnake = 0;
-            if (act && st >= 0) {
-                if (sl == 0) {
-                    S.status = st;
-                    S.used = S.navail = navail;
-                    S.dif = dif;
-                    S.a = a;
-                    S.b = b;
-                    S.ktop = k;   // lane 0's diagonal
-                    S.besta = besta;
-                    S.lasta = lasta;
-                    S.amin = amin;
-                    S.bmax = bmax;
+        if (stop) {
+            if (lane_in(stop)) {
+                int st = LA_OK;
+                if (navail > cap) st = LA_POOL;
+                else if (lane_in(run)) {
+                    if (mk == 0) st = LA_UNDEF;   // empty band with the loop still running
+                    else if (lane_in(aborted)) st = LA_ABORT;
+                    else if (nb - na >= kHalfBand) st = LA_GROW;
+                    else st = LA_UNDEF;
                 }
-                a = na = 1;
-                b = nb = 0;
-                amin = kFar;
-                bmax = -kFar;
+                if (st == LA_GROW) {
+                    D->V[sl] = V;
+                    D->M[sl] = M;
+                    D->HA[sl] = HA;
+                    D->HB[sl] = HB;
+                    D->tA[sl] = tA;
+                    D->tB[sl] = tB;
+                    D->N[sl] = N;
+                }
+                if (sl == 0) {
+                    S->status = st;
+                    S->used = S->navail = navail;
+                    S->dif = dif;
+                    S->a = a;
+                    S->b = b;
+                    S->ktop = k;   // lane 0's diagonal
+                    S->besta = besta;
+                    S->lasta = lasta;
+                    S->amin = amin;
+                    S->bmax = bmax;
+                }
+                na = 1;
+                nb = 0;
                 V = kSentV;
             }
             wave_sync();
-            if (bs & 0xffffffffull) stopped |= 1u;
-            if (bs >> 32) stopped |= 2u;
+            act &= ~stop;
+            if (stop & 0xffffffffull) stopped |= 1u;
+            if (stop >> 32) stopped |= 2u;
         }
         // lanes 0 and 31 stay free: move the band to the middle of its half
-        const bool mv = na < 1 || nb > kHalfBand;
-        if (__any(mv)) {
+        if (ballot(na < 1) | ballot(nb > kHalfBand)) {
+            const bool mv = na < 1 || nb > kHalfBand;
             const int d = mv ? na - (1 + (kHalfBand - (nb - na + 1)) / 2) : 0;   // lane L takes lane L + d
             const int src = lane + d;
             const bool ok = (src >> 5) == (lane >> 5);
@@ -1242,20 +1363,19 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
             na -= d;
             nb -= d;
             k -= d;
-            if (act) {
-                amin -= d;
-                bmax -= d;
-            }
+            amin -= d;
+            bmax -= d;
         }
         dif += 1;
+        fresh = 0;
         a = na;
         b = nb;
 
         // ---- the next wave: predecessors (dalign/align.c:760-791, :1498-1529)
         {
-            const int am = from_above(V), ap = from_below(V);   // k - 1, k + 1
+            const int am = dpp_shl1(V), ap = dpp_shr1(V);   // k - 1, k + 1
             // a new end diagonal takes the thresholds of its inner neighbour
-            const int t0 = lane + ((ea && sl == a) ? 1 : 0) - ((eb && sl == b) ? 1 : 0);
+            const int t0 = lane + (lane_in(ea & ballot(sl == a)) ? 1 : 0) - (lane_in(eb & ballot(sl == b)) ? 1 : 0);
             tA = bperm(tA, t0);
             tB = bperm(tB, t0);
             const int mx = max(am, ap);
@@ -1266,50 +1386,27 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
             HA = bperm(HA, src);
             HB = bperm(HB, src);
             N = bperm64(N, src);
-            V = kSentV;
-            end = false;
-            bool undef = false;
-            if (sl >= a && sl <= b) {
-                y = (c - k) >> 1;
-                const int x = y + k, lim = min(limA - x, limB - y);
-                undef = lim < 0;
-                const int s = max(snake_len(A, B, m, x, y, lim), 0);
-                end = s == lim;
-                nsnake += s + 1;
-                add_columns(N, M, s);
-                y += s;
-                V = 2 * y + k;
-            }
-            const unsigned long long bu = __ballot(undef);
-            if (bu) {
-                const uint32_t mu = hmask(hm, bu);
-                int tc = ncell, ts = nsnake;
-#pragma unroll
-                for (int o = 16; o >= 1; o >>= 1) {
-                    tc += __shfl_xor(tc, o, 64);
-                    ts += __shfl_xor(ts, o, 64);
-                }
-                if (sl == 0) {
-                    S.cells += tc;
-                    S.snake += ts;
-                }
-                ncell = nsnake = 0;
-                if (mu) {
-                    if (sl == 0) {
-                        S.status = LA_UNDEF;
-                        S.used = navail;
-                        S.dif = dif - 1;
-                    }
-                    a = 1;
-                    b = 0;
-                    amin = kFar;
-                    bmax = -kFar;
-                    V = kSentV;
-                    end = false;
+            const Lanes in = ballot(sl >= a) & ballot(sl <= b) & act;
+            y = (c - k) >> 1;
+            const int lim = lane_in(in) ? min(limA - (y + k), limB - y) : 0;
+            const Lanes undef = ballot(lim < 0);
+            const int s = snake_len(A, B, m, y + k, y, lim, lim > 0);
+            rem = lane_in(in) ? lim - s : 1;
+            nsnake += lane_in(in) ? s + 1 : 0;
+            add_columns(N, M, s);
+            y += s;
+            V = lane_in(in) ? 2 * y + k : kSentV;
+            if (undef) {
+                const uint32_t mu = hmask(hm, undef);
+                if (mu && sl == 0) {
+                    S->status = LA_UNDEF;
+                    S->used = navail;
+                    S->dif = dif - 1;
                 }
                 wave_sync();
-                if (bu & 0xffffffffull) stopped |= 1u;
-                if (bu >> 32) stopped |= 2u;
+                act &= ~ballot(mu != 0);
+                if (undef & 0xffffffffull) stopped |= 1u;
+                if (undef >> 32) stopped |= 2u;
             }
         }
     }

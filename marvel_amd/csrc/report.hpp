@@ -258,7 +258,7 @@ struct PairState {
     int novla, novlb, tmin, tmax, touched, band0;
     long long ttop, aligned, edges, cells, snake, steps;
     long long lidx, nidx, h2, f0;   // panel [lidx, nidx), start of the next one, next seed to test
-    int amark2;
+    int amark2, prio;
 };
 
 // (NCH: each kernel has its own copy, so its registers fit that kernel's)
@@ -301,6 +301,7 @@ struct PairJob {
                 if (lane == 0) {
                     const int job = a->order[t], p = a->jobs[job];
                     P.job = job;
+                    P.prio = queue_priority(t, a->norder);
                     P.ps = a->pstart[p];
                     P.pe = a->pstart[p + 1];
                     const Seed s0 = a->hits[P.ps];
@@ -392,6 +393,7 @@ struct PairJob {
         const bool selfie = a->self && !a->comp && P.ar == P.br;
         const int maxtp = 2 * ((P.alen > P.blen ? P.alen : P.blen) / a->tspace + 2);
         uint16_t* latr = a->latr + (size_t)slot * 4 * a->maxtp_all;
+        S.prio = P.prio;
         S.A = a->pkA + a->w0A[P.ar];
         S.B = a->pkB + a->w0B[P.br];
         S.alen = P.alen;

@@ -22,9 +22,9 @@ from .lib import MiTuning, lib
 
 FIELDS = ("report_waves_per_cu", "report_pool_log2", "report_l1_waves_per_cu", "batch_waves_per_cu",
           "batch_wide_waves_per_cu")
-DEFAULT = {"report_waves_per_cu": 20, "report_pool_log2": 15, "report_l1_waves_per_cu": 8, "batch_waves_per_cu": 20,
+DEFAULT = {"report_waves_per_cu": 24, "report_pool_log2": 15, "report_l1_waves_per_cu": 8, "batch_waves_per_cu": 24,
            "batch_wide_waves_per_cu": 4}
-REPORT_CANDIDATES = [(w, p) for w in (12, 16, 20) for p in (14, 15)]
+REPORT_CANDIDATES = [(w, p) for w in (16, 20, 24) for p in (14, 15)]
 L1_CANDIDATES = (4, 8, 12)
 # (first window, 256-diagonal window): the levels are timed apart, so each
 # run scores one candidate of each and the two are chosen independently
