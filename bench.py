@@ -98,7 +98,7 @@ def profiled_traffic(kernel):
 
 
 def profiled_valu_per_wave_step():
-    """VALU instructions per aligner wave step of k_report<1, false> from the committed counter summary
+    """VALU instructions per alignment step of k_report (two alignments per wave) from the committed counter summary
     (SQ_INSTS_VALU per launch over the launch's wave steps).  None when the summary is absent."""
     path = os.path.join(ROOT, "profiles", "k_report_pmc_5mbp.md")
     if not os.path.exists(path):
@@ -226,7 +226,7 @@ def batched_leg(n=2_000_000, seed=3):
                         "seed up to 200 bp off the true diagonal, COMP on half; generated in HBM (seed 3)",
             "value": round(n / t, 1), "unit": "tasks/s", "s_per_batch": round(t, 3),
             "aligned": int(ok.sum()), "undefined_state": int(st[3]), "trace_values": r.used,
-            "roofline": {"bound": "valu", "kernel": "la_batch_kernel (one wave64 per task, persistent queue)",
+            "roofline": {"bound": "valu", "kernel": "la_batch_kernel (two tasks per wave64, persistent queue)",
                          "achieved": round(ach, 2), "peak": VALU_PEAK_GOPS, "unit": "Gop/s (W_align lane-ops)",
                          "frac": round(ach / VALU_PEAK_GOPS, 5), "w_align": w_alg,
                          "kernel_s": round(kern_s, 4), "kernel_s_per_level": [x / 1e6 for x in r.work[2:6]],
@@ -517,10 +517,10 @@ def main():
             "parity": "bit-exact vs reference daligner" if ok else f"MISMATCH sha256 {sha}",
             "pcie_inclusive": {"value": round(n / t_pcie, 1), "unit": "overlaps/s", "ms_per_step": round(t_pcie * 1e3, 2),
                                "note": "one step whose index build uploads the block's reads from host memory"},
-            "roofline": {"bound": "valu", "kernel": "k_report (one wave64 per read pair: gating + Local_Alignment)",
+            "roofline": {"bound": "valu", "kernel": "k_report (two read pairs per wave64: gating + Local_Alignment)",
                          "achieved": round(ach, 2), "peak": VALU_PEAK_GOPS, "unit": "Gop/s (W_align lane-ops)",
                          "frac": round(ach / VALU_PEAK_GOPS, 5), "traffic": profiled_traffic("k_report<1, false>"),
-                         "traffic_unit": "HBM bytes per k_report<1, false> launch (rocprofv3 --pmc, calibrated)",
+                         "traffic_unit": "HBM bytes per launch of the one-alignment-per-wave k_report (rocprofv3 --pmc, calibrated)",
                          "kernel_ms_per_step": round(k_report * 1e3, 2), "launches_per_step": launches,
                          "w_align_per_step": w_align, "issue": issue},
             "roofline_hbm": {"bound": "hbm", "kernel": "seed LSD radix sort (rs_hist + rs_scatter)",
