@@ -1,0 +1,58 @@
+"""The batched aligner's device code on the CPU (tests/wave_emu) against the
+oracle: the kernels of marvel_amd/csrc/la_pack.hpp and la_batch_core.hpp
+compiled by g++, one fiber per lane."""
+
+import os
+import shutil
+
+import numpy as np
+import pytest
+
+import emu_lib
+import la_golden
+import oracle_lib
+from marvel_amd import latasks
+from marvel_amd.align import la_batch
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None or os.uname().machine != "x86_64",
+                                reason="needs g++ on x86-64")
+
+
+@pytest.fixture(scope="module", params=[False, True], ids=["", "garbage"])
+def emu(request):
+    """One library as built, one whose LDS holds garbage when a kernel starts."""
+    os.environ.setdefault("MI_EMU_CUS", "1")
+    emu_lib.build()
+    return emu_lib.Lib(request.param)
+
+
+def check(emu, ts):
+    """Every task the oracle defines is its result, every other one status 3; returns the number of the former."""
+    want, st = oracle_lib.run_tasks(ts)
+    with emu_lib.in_place_of_gpu(emu):
+        got, status = la_batch(ts)
+    keep = [i for i in range(ts.n) if st[i] == 0]
+    bad = la_golden.diff([got[i] for i in keep], [want[i] for i in keep], status[keep])
+    assert not bad, "\n".join(bad)
+    assert all(status[i] == 3 for i in range(ts.n) if st[i] != 0)
+    return len(keep)
+
+
+@pytest.mark.parametrize("tspace,offmax,emax", [(100, 5, 0.25), (100, 60, 0.25), (100, 200, 0.2), (126, 5, 0.12),
+                                                (13, 5, 0.12)])
+def test_noisy_pairs(emu, tspace, offmax, emax):
+    assert check(emu, latasks.make_tasks(20, tspace + offmax, lmin=300, lmax=2500, emin=0.02, emax=emax,
+                                         offmax=offmax, tspace=tspace)) >= 14
+
+
+def test_one_task_leaves_half_the_wave_idle(emu):
+    check(emu, latasks.make_tasks(1, 5, lmin=800, lmax=1500, emin=0.1, emax=0.2, offmax=0))
+
+
+@pytest.mark.parametrize("width", [2, 30, 31, 90])
+def test_initial_bands(emu, width):
+    ts = latasks.make_tasks(6, 300 + width, lmin=1500, lmax=2500, emin=0.05, emax=0.15, offmax=0)
+    par = ts.par.copy()
+    par[:, 3] -= width // 2
+    par[:, 4] = par[:, 3] + width - 1
+    check(emu, latasks.TaskSet(ts.ave_corr, ts.tspace, ts.freq, ts.reads, par.astype(np.int32)))

@@ -8,6 +8,7 @@
 //   * hipLaunchKernelGGL runs the grid's blocks one after another, each block
 //     with one host thread per work-item; __syncthreads is a barrier over the
 //     block, __shared__ arrays are function statics (blocks never overlap);
+//     with MI_EMU_FIBERS the work-items are fibers of one thread;
 //   * the wave64 cross-lane operations of wave_emu.hpp need blocks of 64
 //     work-items (one wave), the only shape the kernels use them in.
 // Streams are synchronous and every API call succeeds unless memory runs out.
@@ -24,6 +25,7 @@
 
 #define __launch_bounds__(...)
 #define __shared__ static
+#define __align__(n) __attribute__((aligned(n)))
 #define HIP_KERNEL_NAME(...) __VA_ARGS__
 
 struct dim3 {
@@ -32,9 +34,13 @@ struct dim3 {
 };
 
 namespace emu {
-extern thread_local dim3 t_block, t_thread;
+extern EMU_LANE_LOCAL dim3 t_block, t_thread;
 extern dim3 g_bdim, g_gdim;
 extern YieldBarrier* g_blockbar;
+#ifdef MI_EMU_FIBERS
+// runs work(t) for t = 0 .. nt - 1, each on a fiber; set(t) before a fiber goes on
+void run_fibers(unsigned nt, const std::function<void(unsigned)>& set, const std::function<void(unsigned)>& work);
+#endif
 
 template <class F>
 void launch(dim3 grid, dim3 block, F&& body)
@@ -49,20 +55,30 @@ void launch(dim3 grid, dim3 block, F&& body)
     g_blockbar = &bar;
     g_bdim = block;
     g_gdim = grid;
+    auto set = [&](unsigned t) {
+        lane = (int)(t & 63);
+        g = nw ? &ctx[t / 64] : nullptr;
+        t_thread = dim3(t, 0, 0);
+    };
+    auto work = [&](unsigned) {
+        for (unsigned b = 0; b < nb; b++) {
+            t_block = dim3(b, 0, 0);
+            body();
+            bar.arrive_and_wait();
+        }
+    };
+#ifdef MI_EMU_FIBERS
+    run_fibers(nt, set, work);
+#else
     std::vector<std::thread> th;
     th.reserve(nt);
     for (unsigned t = 0; t < nt; t++)
         th.emplace_back([&, t] {
-            lane = (int)(t & 63);
-            g = nw ? &ctx[t / 64] : nullptr;
-            t_thread = dim3(t, 0, 0);
-            for (unsigned b = 0; b < nb; b++) {
-                t_block = dim3(b, 0, 0);
-                body();
-                bar.arrive_and_wait();
-            }
+            set(t);
+            work(t);
         });
     for (auto& x : th) x.join();
+#endif
     g = saved;
 }
 }  // namespace emu
@@ -73,7 +89,7 @@ void launch(dim3 grid, dim3 block, F&& body)
 #define gridDim emu::g_gdim
 #define __syncthreads() emu::g_blockbar->arrive_and_wait()
 namespace emu {
-extern thread_local const void* t_kernarg;
+extern EMU_LANE_LOCAL const void* t_kernarg;
 // a kernel called with copies of its arguments; the first one's address
 // stands for the kernarg segment (kernels that read their arguments there)
 template <class F, class A0, class... As>
@@ -165,6 +181,12 @@ inline hipError_t hipMemset(void* d, int v, size_t n)
     return hipSuccess;
 }
 inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t = nullptr) { return hipMemset(d, v, n); }
+#define HIP_SYMBOL(x) ((void*)&(x))
+inline hipError_t hipGetSymbolAddress(void** d, void* sym)
+{
+    *d = sym;
+    return hipSuccess;
+}
 inline hipError_t hipStreamCreate(hipStream_t* s)
 {
     *s = (hipStream_t)0x1;

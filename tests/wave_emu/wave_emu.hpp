@@ -4,6 +4,9 @@
 // debugged on the CPU.  Every cross-lane operation is a two-phase barrier
 // exchange, so all 64 lanes must reach the same sequence of them (true for
 // the aligner: its cross-lane operations sit in wave-uniform control flow).
+// With MI_EMU_FIBERS the lanes are fibers of one host thread (x86-64): a
+// barrier switches stacks instead of threads, about 50 times faster, for test
+// sets; AddressSanitizer needs the threads.
 #pragma once
 #include <sched.h>
 
@@ -18,7 +21,18 @@
 #define __noinline__ __attribute__((noinline))
 #define __host__
 
+#ifdef MI_EMU_FIBERS
+#define EMU_LANE_LOCAL   // one host thread: set at every switch (emu_runtime.cpp)
+#else
+#define EMU_LANE_LOCAL thread_local
+#endif
+
 namespace emu {
+#ifdef MI_EMU_FIBERS
+void lane_yield();
+#else
+inline void lane_yield() { sched_yield(); }
+#endif
 // Generation barrier that yields while waiting: the lanes outnumber the host
 // cores, and a yield hands the core to a lane that has not arrived yet.
 struct YieldBarrier {
@@ -33,15 +47,15 @@ struct YieldBarrier {
             count.store(0, std::memory_order_relaxed);
             gen.fetch_add(1, std::memory_order_acq_rel);
         } else
-            while (gen.load(std::memory_order_acquire) == g0) sched_yield();
+            while (gen.load(std::memory_order_acquire) == g0) lane_yield();
     }
 };
 struct Ctx {
     YieldBarrier bar{64};
     long long slot[64];
 };
-extern thread_local Ctx* g;   // the calling lane's wave
-extern thread_local int lane;
+extern EMU_LANE_LOCAL Ctx* g;   // the calling lane's wave
+extern EMU_LANE_LOCAL int lane;
 template <class T>
 inline T xchg(T v, int src)
 {
