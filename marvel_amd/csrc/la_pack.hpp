@@ -31,7 +31,7 @@
 //   * What the reference tests against memory is carried instead: a
 //     diagonal's trace-point thresholds and its pebbles' trace points as
 //     small numbers (the 8 low bits of the number ride on the pebble's
-//     index), so a wave that crosses trace points only stores; the
+//     index, see skip_points), so a wave that crosses trace points only stores; the
 //     suffix-positivity test of the trim point (dalign/align.c:884-896) reads
 //     a 10-bit table in LDS three times instead of a 128 KB table twice.
 //   * What only changes at events lives in LDS, written by the lane that owns
@@ -342,6 +342,31 @@ __device__ __forceinline__ void pack_tables(PackLds& L, const DevSpec& sp)
     wave_sync();
 }
 
+// ---- many trace points in one wave ------------------------------------------------------
+// A diagonal whose path reached trace point t (those below t are done) pushes a
+// pebble there unless the path's pebble lies at or beyond t.  The 8 low bits
+// of the pebble's number settle that while it lies less than 128 points beyond
+// t (it is never more than one before t).  A diagonal takes a neighbour's
+// path one wave after the neighbour got there and had by then, at least, come
+// as far as the neighbour one wave earlier; so the pebble lies at most as many
+// points beyond t as some diagonal passed in the wave before.  That is 128 or
+// more only in an exact run of that length: both neighbours of a diagonal run
+// through a tandem repeat in one wave, the diagonal itself stays.  So only a
+// wave after one that passed kManyPoints points looks at the paths that end
+// that many points beyond t (a pebble lies on its path), and reads the marks of
+// their pebbles.  (Looking in every wave that crosses trace points cost 2.7 %
+// on the 5 Mbp block, 172.9 -> 177.7 ms a pass.)
+constexpr int kManyPoints = 120;
+constexpr unsigned kMany = 4;          // beside the halves to serve: the last wave passed many points
+__device__ __forceinline__ int many_points(int TS) { return TS <= INT32_MAX / kManyPoints ? kManyPoints * TS : INT32_MAX; }
+// The first point from t on that lies beyond pebble h (point n lies at n TS + off): no point before it needs a pebble.
+__device__ __forceinline__ int skip_points(const Glob<Int4>* pool, int h, int t, int TS, int off, int m)
+{
+    const int p = ((pool[h & kPebIdx][3] ^ m) - m) - off;   // the pebble's mark, in the pass's direction
+    const int n = p / TS;
+    return max(t, n - (n * TS > p ? 1 : 0) + 1);
+}
+
 // ---- a pass over the whole wave -----------------------------------------------------
 // Takes the pass of slot h after the trim of a wave (its diagonals in L->band[h],
 // lanes slot.a .. slot.b) and runs it with 64 NCH diagonals until its
@@ -376,7 +401,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
     int V[NCH], M[NCH], HA[NCH], HB[NCH], tA[NCH], tB[NCH], y[NCH];
     uint64_t N[NCH];
     bool end[NCH];
-    bool fresh = dif < 0, undef = false;
+    bool fresh = dif < 0, undef = false, many = true;
     if (fresh) {   // wave 0 (dalign/align.c:455-587)
         const int hi = uni(S.hgh), wd = hi - uni(S.low) + 1, mida = uni(S.anti);
         const int minp = uni(S.minp), maxp = uni(S.maxp);
@@ -668,7 +693,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
         fresh = false;
         // ---- trace-point pebbles (dalign/align.c:826-878, :1562-1612)
         bool full = false;
-        for (;;) {
+        for (int n = 0;; n++) {   // n: points passed
             bool any = false;
             bool wA[NCH], wB[NCH];
 #pragma unroll
@@ -679,7 +704,31 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 wB[j] = in && y[j] >= mul24(tB[j], TS) + offB;
                 any |= wA[j] | wB[j];
             }
-            if (!any_lane(any)) break;
+            if (!any_lane(any)) {
+                many = n >= kManyPoints;
+                break;
+            }
+            if (many) {   // (see skip_points)
+                const int far = many_points(TS);
+                bool fA[NCH], fB[NCH], f = false;
+#pragma unroll
+                for (int j = 0; j < NCH; j++) {
+                    fA[j] = wA[j] && y[j] + kt - (64 * j + lane) - mul24(tA[j], TS) >= far;
+                    fB[j] = wB[j] && y[j] - mul24(tB[j], TS) - offB >= far;
+                    f |= fA[j] | fB[j];
+                }
+                many = false;
+                if (any_lane(f)) {
+                    wave_sync();   // pebbles of this wave's other lanes
+#pragma unroll
+                    for (int j = 0; j < NCH; j++) {
+                        if (fA[j]) tA[j] = skip_points(pool, HA[j], tA[j], TS, 0, m);
+                        if (fB[j]) tB[j] = skip_points(pool, HB[j], tB[j], TS, offB, m);
+                    }
+                    n = kManyPoints;
+                    continue;
+                }
+            }
 #pragma unroll
             for (int j = 0; j < NCH; j++) {
                 if (!live(j)) continue;
@@ -1036,13 +1085,36 @@ static __device__ __noinline__ void pass_begin(PackLds* L, int h)
     wave_sync();
 }
 
+// The trace points that the paths in the PackBands have already are done;
+// whether there were any.
+static __device__ __noinline__ bool pack_skip(PackLds* L)
+{
+    const int lane = __lane_id(), sl = lane & 31;
+    const PackSlot& S = L->slot[lane >> 5];
+    PackBand& D = L->band[lane >> 5];
+    const int TS = uni(L->sp.tspace), far = many_points(TS);
+    const int m = S.phase == PH_REV ? -1 : 0;
+    const int offB = ((S.comp ? S.blen % TS : 0) ^ m) - m;
+    const int k = S.ktop - sl, y = (D.V[sl] - k) >> 1, tA = D.tA[sl], tB = D.tB[sl];
+    const bool in = sl >= S.a && sl <= S.b;
+    const bool fA = in && y + k - mul24(tA, TS) >= far, fB = in && y - offB - mul24(tB, TS) >= far;
+    wave_sync();   // pebbles of the wave's other lanes
+    Glob<Int4>* pool = (Glob<Int4>*)S.pool;
+    if (fA) D.tA[sl] = skip_points(pool, D.HA[sl], tA, TS, 0, m);
+    if (fB) D.tB[sl] = skip_points(pool, D.HB[sl], tB, TS, offB, m);
+    wave_sync();
+    return any_lane(fA || fB);
+}
+
 // The halves in `stopped` (bit 0: lanes 0..31): a pass that needs the wave
 // gets it, one that ended is followed by the next.  Afterwards every slot
 // holds a pass that goes on from its PackBand, or is idle with an empty band.
+// kMany in `stopped`, and a pass back from wide_run: pack_skip.  Returns kMany where the next wave needs it again.
 template <int NCH, class Job>
-__device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, const int* abort_flag)
+__device__ __noinline__ unsigned pack_serve(Job job, PackLds* L, unsigned stopped, const int* abort_flag)
 {
     const int lane = __lane_id();
+    bool many = (stopped & kMany) != 0;
     for (int h = 0; h < 2; h++) {
         if (!((stopped >> h) & 1)) continue;
         PackSlot& S = L->slot[h];
@@ -1051,6 +1123,7 @@ __device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, c
             if (uni(S.phase) != PH_IDLE && uni(S.status) == LA_GROW) {
                 wide_run<NCH>(L, h, abort_flag);
                 go = uni(S.running) != 0;
+                many |= go;
                 if (lane == 0) {
                     S.running = 0;
                     if (go) S.status = LA_OK;
@@ -1075,6 +1148,7 @@ __device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, c
         }
     }
     set_priority(max(uni(L->slot[0].prio), uni(L->slot[1].prio)));
+    return many && pack_skip(L) ? kMany : 0;
 }
 
 // ---- the loop --------------------------------------------------------------------------
@@ -1103,7 +1177,7 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
     int ncell = 0, nsnake = 0;
     // wave-uniform
     Lanes act = 0, fresh = 0;                // halves with a pass; of these, in wave 0
-    unsigned stopped = second ? 3u : 1u;     // halves to serve (bit 0: lanes 0..31)
+    unsigned stopped = second ? 3u : 1u;     // halves to serve (bit 0: lanes 0..31), kMany
     unsigned tick = 0;
 
     for (;;) {
@@ -1141,8 +1215,7 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
                 }
             }
             wave_sync();
-            pack_serve<NCH>(job, &L, stopped, abort_flag);
-            stopped = 0;
+            stopped = (unsigned)uni((int)pack_serve<NCH>(job, &L, stopped, abort_flag));
             lane = __lane_id();
 #ifndef MI_CPU_WAVE_EMU
             asm volatile("" : "+v"(lane));   // computed here, not once before the loop
@@ -1201,7 +1274,7 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
             int nA = mul24(tA, TS), nB = mul24(tB, TS) + offB;
             const Lanes in = ballot(sl >= a) & ballot(sl <= b);
             Lanes wA = in & ballot(x >= nA), wB = in & ballot(y >= nB);
-            while (wA | wB) {
+            if (wA | wB) for (int n = 1;; n++) {   // n: points passed
                 const Lanes pA = wA & (fresh | ballot((int)(((unsigned)tA << 24) - ((unsigned)HA & ~(unsigned)kPebIdx)) > 0));
                 const Lanes pB = wB & (fresh | ballot((int)(((unsigned)tB << 24) - ((unsigned)HB & ~(unsigned)kPebIdx)) > 0));
                 const int al = __popcll(pA & 0xffffffffull), bl = __popcll(pB & 0xffffffffull);
@@ -1225,6 +1298,8 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
                 nB = mul24(tB, TS) + offB;
                 wA &= ballot(x >= nA);
                 wB &= ballot(y >= nB);
+                if (!(wA | wB)) break;
+                if (n == kManyPoints - 1) stopped = kMany;
             }
         }
 

@@ -13,6 +13,7 @@ import pytest
 
 import las_cases
 import oracle_lib
+import repeat_tasks
 from marvel_amd import dbio
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -321,3 +322,23 @@ def test_tuning_keeps_output(tmp_path):
     for i in range(dt.n):
         assert np.array_equal(ta[a["atrace"][i]:a["atrace"][i] + a["atlen"][i]],
                               tb[b["atrace"][i]:b["atrace"][i] + b["atlen"][i]]), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seed,tspace,error", [(1, 5, 0.004), (2, 5, 0.004), (1, 10, 0.002)])
+def test_exact_tandem_repeats_in_reads(tmp_path, seed, tspace, error):
+    """Reads with exact tandem repeats of 130 to 300 trace spacings: the .las
+    is the oracle's (the first set's was not while a pebble's trace point was
+    compared by 8 bits of its number alone)."""
+    oracle_lib.ensure_built()
+    print(f"[gpu daligner] exact repeats seed={seed} -s{tspace}", flush=True)
+    got = []
+    for exe in (EXE, oracle_lib.ORACLE_CLI):
+        d = str(tmp_path / os.path.basename(exe))
+        os.makedirs(d)
+        dbio.write_db(os.path.join(d, "S"), repeat_tasks.reads(seed, tspace, error), size_mbp=400)
+        r = subprocess.run([exe, "-j4", "-M8", f"-s{tspace}", "S.1", "S.1"], cwd=d, capture_output=True, text=True,
+                           timeout=240)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(_shas(d))
+    assert got[0] == got[1] and len(got[0]) > 0

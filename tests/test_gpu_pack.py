@@ -3,14 +3,16 @@ at the sizes where its paths change, against the oracle: batches that leave
 the upper halves idle and batches that use them, bands that stay within a
 half's 30 diagonals, that outgrow them for a while, and that outgrow the 128
 diagonals of the first wide window; trace spacings below and above the snake
-step, whose trace-point numbers wrap at 256; and initial bands of several
-diagonals up to and beyond a half."""
+step, whose trace-point numbers wrap at 256; initial bands of several
+diagonals up to and beyond a half; and exact tandem repeats, in which a path
+gets more than 128 or 256 trace points ahead of a diagonal that takes it."""
 
 import numpy as np
 import pytest
 
 import la_golden
 import oracle_lib
+import repeat_tasks
 from marvel_amd import latasks
 from marvel_amd.align import la_batch
 from marvel_amd.lib import MiTuning, lib
@@ -72,3 +74,18 @@ def test_initial_bands(width):
     reads = [r for i in keep for r in (ts.reads[2 * i], ts.reads[2 * i + 1])]
     print(f"[pack] width={width} n={len(keep)}", flush=True)
     _check(latasks.TaskSet(ts.ave_corr, ts.tspace, ts.freq, reads, par[np.array(keep)]))
+
+
+@pytest.mark.parametrize("tspace", [10, 20, 50, 100])
+@pytest.mark.parametrize("width,tail", [(1, 0), (2, 2500), (5, 0), (20, 2500), (40, 0), (150, 2500)])
+def test_exact_tandem_repeats(tspace, width, tail):
+    for points in ((128, 260), (260, 420)):
+        ts = repeat_tasks.make(16, 31 * tspace + width + points[0], tspace, points, width=width, tail=tail)
+        print(f"[pack] repeats tspace={tspace} width={width} points={points} tail={tail}", flush=True)
+        _check(ts)
+
+
+def test_exact_tandem_repeats_on_both_halves(few_waves):
+    ts = repeat_tasks.make(1400, 8, 10, (128, 300), width=5, tail=200, flank=100)
+    print(f"[pack] repeats n={ts.n}", flush=True)
+    _check(ts)

@@ -11,6 +11,7 @@ import pytest
 import emu_lib
 import la_golden
 import oracle_lib
+import repeat_tasks
 from marvel_amd import latasks
 from marvel_amd.align import la_batch
 
@@ -56,3 +57,13 @@ def test_initial_bands(emu, width):
     par[:, 3] -= width // 2
     par[:, 4] = par[:, 3] + width - 1
     check(emu, latasks.TaskSet(ts.ave_corr, ts.tspace, ts.freq, ts.reads, par.astype(np.int32)))
+
+
+@pytest.mark.parametrize("tspace", [5, 20, 100])
+@pytest.mark.parametrize("width,points,tail", [(1, (250, 420), 0), (5, (128, 260), 0), (5, (260, 420), 2500),
+                                               (20, (128, 260), 2500), (40, (260, 420), 0), (150, (128, 300), 0)])
+def test_exact_tandem_repeats(emu, tspace, width, points, tail):
+    """Paths more than 128 and more than 256 trace points ahead of a
+    diagonal's thresholds: a pebble's point is known by 8 bits of its number
+    (far_points, la_pack.hpp)."""
+    check(emu, repeat_tasks.make(6, 1000 * tspace + width + tail, tspace, points, width=width, tail=tail))
