@@ -1084,15 +1084,15 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
     // wider), 256 and 1,024 diagonals; the pools are sized for typical pairs,
     // outliers go to the larger levels; the last also has the large pebble
     // pools and match arenas
-    constexpr int kLevels = 4;
+    constexpr int kLevels = 4, kWideLevel = 2;   // kWideLevel: the first of kWideNch
     const MiTuning& tu = mi_tuning();
     const int l0_waves = cus * (tu.report_waves_per_cu ? tu.report_waves_per_cu : 4 * kPackWaves);
     const int l0_pool = 1 << (tu.report_pool_log2 ? tu.report_pool_log2 : 15);
     const int l1_waves = cus * (tu.report_l1_waves_per_cu ? tu.report_l1_waves_per_cu : 8);
     const Level levels[kLevels] = {{2, l0_pool, 128, 1 << 16, l0_waves},
                                    {4, 1 << 16, 256, 1 << 18, l1_waves},
-                                   {16, 1 << 17, 256, 1 << 18, cus * 4},
-                                   {16, 1 << 20, 4096, 1LL << 22, std::min(cus, 128)}};
+                                   {kWideNch, 1 << 17, 256, 1 << 18, cus * 4},
+                                   {kWideNch, 1 << 20, 4096, 1LL << 22, std::min(cus, 128)}};
     const int small_trace = TS <= TRACE_XOVR ? 1 : 0;
     const int tbytes = small_trace ? 1 : 2;
 
@@ -1216,12 +1216,13 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
     a.hitmin = g_hitmin;
     a.minhit = minhit;
     a.minover = MINOVER;
-    a.tspace = TS;
+    a.tspace = point_spacing(TS, std::max(A->maxlen, B->maxlen));
     a.small_trace = small_trace;
     a.mindiag = mindiag;
     a.maxdiag = maxdiag;
     a.w = w;
     a.sp = ds->spec;
+    a.sp.tspace = a.tspace;
     a.maxtp_all = maxtp_all;
     a.edge_in = edge_in.p;
     a.edge_out = edge_out.p;
@@ -1292,7 +1293,7 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
         switch (L.nch) {
         case 2: launch_report<2>(b, grid); break;
         case 4: launch_report<4>(b, grid); break;
-        default: launch_report<16>(b, grid); break;
+        default: launch_report<kWideNch>(b, grid); break;
         }
         HC(hipGetLastError());
         g_ev_report.record_stop();
@@ -1350,6 +1351,7 @@ static void match_pass(KIdx* A, KIdx* B, bool self, int comp, bool same_index, S
     int first_level = 0;
     if (const char* e = getenv("MI_REPORT_FIRST_LEVEL"))
         first_level = std::min(std::max(atoi(e), 0), kLevels - 1);
+    if (!points24(a.tspace, std::max(A->maxlen, B->maxlen))) first_level = std::max(first_level, kWideLevel);
     auto run_all = [&](const int* dorder, long long n) {
         int level = first_level;
         std::vector<std::pair<int, int>> again = run(dorder, n, level);

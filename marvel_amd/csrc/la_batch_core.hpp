@@ -267,6 +267,7 @@ struct Level {
     int pool_cap;
     int waves;   // upper bound; the scratch may cap it
 };
+constexpr int kWideLevel = 2;   // the first level of kWideNch
 constexpr int kSlots = 2;   // alignments a wave holds, each with its own scratch
 
 static const int kCounterBytes = 4096;   // 256 bytes of counters, then the length classes of a queue
@@ -312,7 +313,7 @@ static int launch_level(int nch, int grid, const MiLaTask* tasks, const int* ord
     switch (nch) {
     case 2: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<2>), dim3(grid), dim3(64), 0, st, a); break;
     case 4: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<4>), dim3(grid), dim3(64), 0, st, a); break;
-    case 16: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<16>), dim3(grid), dim3(64), 0, st, a); break;
+    case kWideNch: hipLaunchKernelGGL(HIP_KERNEL_NAME(la_batch_kernel<kWideNch>), dim3(grid), dim3(64), 0, st, a); break;
     default: return -1;
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -341,8 +342,8 @@ static BatchPlan make_plan(int maxlen, int tspace, int cus)
     // next level when its band outgrows the window or its pool fills
     p.lv[0] = Level{2, 1 << 15, cus * (w0 ? w0 : 4 * kPackWaves)};
     p.lv[1] = Level{4, 1 << 17, cus * (w1 ? w1 : 4)};
-    p.lv[2] = Level{16, 1 << 18, 256};
-    p.lv[3] = Level{16, 1 << 20, 256};
+    p.lv[kWideLevel] = Level{kWideNch, 1 << 18, 256};
+    p.lv[3] = Level{kWideNch, 1 << 20, 256};
     return p;
 }
 
@@ -368,7 +369,7 @@ static int check_tasks(const MiLaTask* d_tasks, int ntasks, long long npacked, i
 
 // The level loop.  `area` holds the counters, the retry lists and the
 // per-level wave scratch; levels whose full grid does not fit run fewer waves.
-static int run_batch(const DevSpec& sp, const uint64_t* pk, const MiLaTask* tasks, int ntasks, int maxlen,
+static int run_batch(DevSpec sp, const uint64_t* pk, const MiLaTask* tasks, int ntasks, int maxlen,
                      const int* order, MiLaResult* res, uint16_t* arena, long long arena_cap,
                      unsigned long long* d_arena_top, const ScratchArea& area, const int* abort_flag, bool watchdog,
                      long long* work, const char* who)
@@ -398,10 +399,12 @@ static int run_batch(const DevSpec& sp, const uint64_t* pk, const MiLaTask* task
             if (ev[i] == nullptr && hipEventCreate(&ev[i]) != hipSuccess) return MI_ERR_DEVICE;
     }
     const BatchPlan plan = make_plan(maxlen, sp.tspace, mi_num_cus());
+    sp.tspace = point_spacing(sp.tspace, maxlen);
+    const int first = points24(sp.tspace, maxlen) ? 0 : kWideLevel;
     const int* cur = order;
     int n = ntasks;
     int which = 0;
-    for (int level = 0; level < 4 && n > 0; level++) {
+    for (int level = first; level < 4 && n > 0; level++) {
         const Level& L = plan.lv[level];
         const size_t per = kSlots * wave_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap) + 3 * 256;
         long long g = std::min<long long>(L.waves, n);
@@ -414,7 +417,7 @@ static int run_batch(const DevSpec& sp, const uint64_t* pk, const MiLaTask* task
         }
         const BatchScratch ws = carve(area.base + fixed, kSlots * (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap);
         int* retry = lists[which];
-        if (level == 0 && cur == nullptr && n > g) {
+        if (level == first && cur == nullptr && n > g) {
             // (the second list is free until the next level's retries)
             int* cls = (int*)(area.base + 256);
             const dim3 nb((n + 255) / 256), bt(256);

@@ -188,14 +188,22 @@ __device__ __forceinline__ KernArgs<T>* kern_args(const T* p)
     return (KernArgs<T>*)uni(p);
 }
 // product of two factors below 2^23 (full rate; the 32-bit multiply takes four times as long)
-__device__ __forceinline__ int mul24(int x, int y)
+__device__ __forceinline__ int mul24(int x, int y) { return __mul24(x, y); }
+// Trace point t's place is t TS, in the narrower windows a 24-bit product.
+// The hosts keep its factors below 2^23 there: point_spacing takes a spacing
+// beyond every read down (no read has a point then, whatever the spacing), and
+// what points24 still refuses -- reads of 2^23 bases or more -- starts at the
+// widest window, whose kernel multiplies in 32 bits.
+constexpr int kMul24 = 1 << 23;
+constexpr int kWideNch = 16;
+template <int NCH>
+__device__ __forceinline__ int point_at(int t, int TS)
 {
-#ifndef MI_CPU_WAVE_EMU
-    return __mul24(x, y);
-#else
-    return x * y;
-#endif
+    if constexpr (NCH == kWideNch) return t * TS;
+    else return mul24(t, TS);
 }
+static inline int point_spacing(int TS, int maxlen) { return TS >= kMul24 && maxlen < kMul24 - 1 ? kMul24 - 1 : TS; }
+static inline bool points24(int TS, int maxlen) { return TS < kMul24 && maxlen / TS + 2 < kMul24; }
 // value of lane `src`
 __device__ __forceinline__ int bperm(int v, int src) { return __builtin_amdgcn_ds_bpermute(src << 2, v); }
 __device__ __forceinline__ uint64_t bperm64(uint64_t v, int src)
@@ -700,8 +708,8 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
             for (int j = 0; j < NCH; j++) {
                 const int i = 64 * j + lane;
                 const bool in = i >= a && i <= b;
-                wA[j] = in && y[j] + kt - i >= mul24(tA[j], TS);
-                wB[j] = in && y[j] >= mul24(tB[j], TS) + offB;
+                wA[j] = in && y[j] + kt - i >= point_at<NCH>(tA[j], TS);
+                wB[j] = in && y[j] >= point_at<NCH>(tB[j], TS) + offB;
                 any |= wA[j] | wB[j];
             }
             if (!any_lane(any)) {
@@ -713,8 +721,8 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 bool fA[NCH], fB[NCH], f = false;
 #pragma unroll
                 for (int j = 0; j < NCH; j++) {
-                    fA[j] = wA[j] && y[j] + kt - (64 * j + lane) - mul24(tA[j], TS) >= far;
-                    fB[j] = wB[j] && y[j] - mul24(tB[j], TS) - offB >= far;
+                    fA[j] = wA[j] && y[j] + kt - (64 * j + lane) - point_at<NCH>(tA[j], TS) >= far;
+                    fB[j] = wB[j] && y[j] - point_at<NCH>(tB[j], TS) - offB >= far;
                     f |= fA[j] | fB[j];
                 }
                 many = false;
@@ -1087,7 +1095,8 @@ static __device__ __noinline__ void pass_begin(PackLds* L, int h)
 
 // The trace points that the paths in the PackBands have already are done;
 // whether there were any.
-static __device__ __noinline__ bool pack_skip(PackLds* L)
+template <int NCH>
+__device__ __noinline__ bool pack_skip(PackLds* L)
 {
     const int lane = __lane_id(), sl = lane & 31;
     const PackSlot& S = L->slot[lane >> 5];
@@ -1097,7 +1106,7 @@ static __device__ __noinline__ bool pack_skip(PackLds* L)
     const int offB = ((S.comp ? S.blen % TS : 0) ^ m) - m;
     const int k = S.ktop - sl, y = (D.V[sl] - k) >> 1, tA = D.tA[sl], tB = D.tB[sl];
     const bool in = sl >= S.a && sl <= S.b;
-    const bool fA = in && y + k - mul24(tA, TS) >= far, fB = in && y - offB - mul24(tB, TS) >= far;
+    const bool fA = in && y + k - point_at<NCH>(tA, TS) >= far, fB = in && y - offB - point_at<NCH>(tB, TS) >= far;
     wave_sync();   // pebbles of the wave's other lanes
     Glob<Int4>* pool = (Glob<Int4>*)S.pool;
     if (fA) D.tA[sl] = skip_points(pool, D.HA[sl], tA, TS, 0, m);
@@ -1148,7 +1157,7 @@ __device__ __noinline__ unsigned pack_serve(Job job, PackLds* L, unsigned stoppe
         }
     }
     set_priority(max(uni(L->slot[0].prio), uni(L->slot[1].prio)));
-    return many && pack_skip(L) ? kMany : 0;
+    return many && pack_skip<NCH>(L) ? kMany : 0;
 }
 
 // ---- the loop --------------------------------------------------------------------------
@@ -1271,7 +1280,7 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
         // (dalign/align.c:521-563, :826-878, :1258-1297, :1562-1612)
         {
             const int x = y + k;
-            int nA = mul24(tA, TS), nB = mul24(tB, TS) + offB;
+            int nA = point_at<NCH>(tA, TS), nB = point_at<NCH>(tB, TS) + offB;
             const Lanes in = ballot(sl >= a) & ballot(sl <= b);
             Lanes wA = in & ballot(x >= nA), wB = in & ballot(y >= nB);
             if (wA | wB) for (int n = 1;; n++) {   // n: points passed
@@ -1294,8 +1303,8 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
                 }
                 tA += lane_in(wA) ? 1 : 0;
                 tB += lane_in(wB) ? 1 : 0;
-                nA = mul24(tA, TS);
-                nB = mul24(tB, TS) + offB;
+                nA = point_at<NCH>(tA, TS);
+                nB = point_at<NCH>(tB, TS) + offB;
                 wA &= ballot(x >= nA);
                 wB &= ballot(y >= nB);
                 if (!(wA | wB)) break;

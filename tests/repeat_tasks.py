@@ -1,4 +1,5 @@
-"""Local_Alignment tasks over long exact tandem repeats.
+"""Local_Alignment tasks over long exact tandem repeats, and over a very long
+read.
 
 Inside an exact repeat of a short period some diagonals of a band run to its
 end in one wave while the ones between them stay where they are, so a
@@ -61,3 +62,17 @@ def reads(seed: int, tspace: int, error: float, coverage: float = 8.0, length: i
         at += ln + int(rng.integers(500, 900))
     return sim.simulate_reads(g, coverage, 3500.0, 800.0, 2000, seed + 1, p_ins=error * .6, p_del=error * .27,
                               p_sub=error * .13).reads
+
+
+def long_read_task(tspace: int) -> latasks.TaskSet:
+    """A short read against the end of one of 2^23 + 3,000 bases: the numbers
+    of the trace points around the seed are beyond 23 bits at a spacing of 1."""
+    rng = np.random.Generator(np.random.PCG64(4))
+    t = rng.integers(0, 4, 1500, dtype=np.uint8)
+    a, am = latasks.mutate_map(t, rng, 0.03, 0.013, 0.007)
+    b, bm = latasks.mutate_map(t, rng, 0.03, 0.013, 0.007)
+    at = 2**23 + 3000 - len(a) - 100
+    read = np.concatenate([rng.integers(0, 4, at, dtype=np.uint8), a, rng.integers(0, 4, 100, dtype=np.uint8)])
+    x, y = at + int(am[700]), int(bm[700])
+    return latasks.TaskSet(0.70, tspace, (0.25, 0.25, 0.25, 0.25), [read, b],
+                           np.array([[len(read), len(b), 0, x - y, x - y, x + y, -1, -1]], dtype=np.int32))

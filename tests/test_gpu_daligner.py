@@ -342,3 +342,20 @@ def test_exact_tandem_repeats_in_reads(tmp_path, seed, tspace, error):
         assert r.returncode == 0, r.stderr[-2000:]
         got.append(_shas(d))
     assert got[0] == got[1] and len(got[0]) > 0
+
+
+@pytest.mark.gpu
+def test_trace_spacing_beyond_every_read(tmp_path):
+    """-s 1073741824: no read has a trace point; the .las is the oracle's."""
+    oracle_lib.ensure_built()
+    print("[gpu daligner] -s1073741824", flush=True)
+    got = []
+    for exe in (EXE, oracle_lib.ORACLE_CLI):
+        d = str(tmp_path / os.path.basename(exe))
+        os.makedirs(d)
+        dbio.write_db(os.path.join(d, "S"), repeat_tasks.reads(3, 100, 0.05), size_mbp=400)
+        r = subprocess.run([exe, "-j4", "-M8", "-s1073741824", "S.1", "S.1"], cwd=d, capture_output=True, text=True,
+                           timeout=240)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(_shas(d))
+    assert got[0] == got[1] and len(got[0]) > 0

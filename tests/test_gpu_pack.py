@@ -4,8 +4,9 @@ the upper halves idle and batches that use them, bands that stay within a
 half's 30 diagonals, that outgrow them for a while, and that outgrow the 128
 diagonals of the first wide window; trace spacings below and above the snake
 step, whose trace-point numbers wrap at 256; initial bands of several
-diagonals up to and beyond a half; and exact tandem repeats, in which a path
-gets more than 128 or 256 trace points ahead of a diagonal that takes it."""
+diagonals up to and beyond a half; exact tandem repeats, in which a path gets
+more than 128 or 256 trace points ahead of a diagonal that takes it; and
+trace points whose spacing or number is beyond 23 bits."""
 
 import numpy as np
 import pytest
@@ -89,3 +90,16 @@ def test_exact_tandem_repeats_on_both_halves(few_waves):
     ts = repeat_tasks.make(1400, 8, 10, (128, 300), width=5, tail=200, flank=100)
     print(f"[pack] repeats n={ts.n}", flush=True)
     _check(ts)
+
+
+@pytest.mark.parametrize("tspace", [2**23 - 1, 2**23, 9_000_000, 2**30])
+def test_trace_spacings_beyond_24_bits(tspace):
+    ts = latasks.make_tasks(8, 5, lmin=300, lmax=900, emin=0.02, emax=0.2, offmax=20, tspace=tspace)
+    print(f"[pack] tspace={tspace}", flush=True)
+    assert _check(ts) == 8
+
+
+@pytest.mark.parametrize("tspace", [1, 100, 2**24])
+def test_a_read_of_more_than_2_to_23_bases(tspace):
+    print(f"[pack] long read, tspace={tspace}", flush=True)
+    assert _check(repeat_tasks.long_read_task(tspace)) == 1

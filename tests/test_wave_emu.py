@@ -14,6 +14,7 @@ import oracle_lib
 import repeat_tasks
 from marvel_amd import latasks
 from marvel_amd.align import la_batch
+from repeat_tasks import long_read_task
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None or os.uname().machine != "x86_64",
                                 reason="needs g++ on x86-64")
@@ -67,3 +68,14 @@ def test_exact_tandem_repeats(emu, tspace, width, points, tail):
     diagonal's thresholds: a pebble's point is known by 8 bits of its number
     (far_points, la_pack.hpp)."""
     check(emu, repeat_tasks.make(6, 1000 * tspace + width + tail, tspace, points, width=width, tail=tail))
+
+
+@pytest.mark.parametrize("tspace", [2**23 - 1, 2**23, 9_000_000, 2**30])
+def test_trace_spacings_beyond_24_bits(emu, tspace):
+    """Trace points are placed by 24-bit products (point_at, la_pack.hpp)."""
+    assert check(emu, latasks.make_tasks(8, 5, lmin=300, lmax=900, emin=0.02, emax=0.2, offmax=20, tspace=tspace)) == 8
+
+
+@pytest.mark.parametrize("tspace", [1, 2, 100, 2**23, 2**24])
+def test_a_read_of_more_than_2_to_23_bases(emu, tspace):
+    assert check(emu, long_read_task(tspace)) == 1

@@ -162,3 +162,5 @@ inline unsigned __builtin_bitreverse32(unsigned x)
     return r;
 }
 inline int __popc(unsigned x) { return __builtin_popcount(x); }
+// v_mul_i32_i24: the low 24 bits of both factors, signed
+inline int __mul24(int x, int y) { return (int)((long long)((x << 8) >> 8) * ((y << 8) >> 8)); }
