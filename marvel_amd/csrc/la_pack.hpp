@@ -382,12 +382,15 @@ __device__ __forceinline__ int skip_points(const Glob<Int4>* pool, int h, int t,
 // their wave's trace points and records) or it ends (running = 0, status).
 // slot.dif < 0: the pass begins here, a forward pass from more diagonals than
 // a half holds.
+// many: whether the wave before the first passed many trace points; returned
+// for the wave before the one the pass goes on with.
 // Index i of the window (lane i & 63 of chunk i >> 6) holds diagonal kt - i.
 template <int NCH>
-__device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
+__device__ __noinline__ int wide_run(PackLds* L, int h, const int* abort_flag, int many)
 {
     constexpr int W = 64 * NCH;
     const int lane = __lane_id();
+    many = uni(many);
     PackSlot& S = L->slot[h];
     PackHot& H = L->hot[h];
     PackBand& D = L->band[h];
@@ -409,7 +412,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
     int V[NCH], M[NCH], HA[NCH], HB[NCH], tA[NCH], tB[NCH], y[NCH];
     uint64_t N[NCH];
     bool end[NCH];
-    bool fresh = dif < 0, undef = false, many = true;
+    bool fresh = dif < 0, undef = false;
     if (fresh) {   // wave 0 (dalign/align.c:455-587)
         const int hi = uni(S.hgh), wd = hi - uni(S.low) + 1, mida = uni(S.anti);
         const int minp = uni(S.minp), maxp = uni(S.maxp);
@@ -713,7 +716,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                 any |= wA[j] | wB[j];
             }
             if (!any_lane(any)) {
-                many = n >= kManyPoints;
+                many = n >= kManyPoints ? 1 : 0;
                 break;
             }
             if (many) {   // (see skip_points)
@@ -725,7 +728,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
                     fB[j] = wB[j] && y[j] - point_at<NCH>(tB[j], TS) - offB >= far;
                     f |= fA[j] | fB[j];
                 }
-                many = false;
+                many = 0;
                 if (any_lane(f)) {
                     wave_sync();   // pebbles of this wave's other lanes
 #pragma unroll
@@ -882,6 +885,7 @@ __device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
         }
     }
     wave_sync();
+    return many;
 }
 
 // ---- between passes ------------------------------------------------------------------
@@ -1118,21 +1122,20 @@ __device__ __noinline__ bool pack_skip(PackLds* L)
 // The halves in `stopped` (bit 0: lanes 0..31): a pass that needs the wave
 // gets it, one that ended is followed by the next.  Afterwards every slot
 // holds a pass that goes on from its PackBand, or is idle with an empty band.
-// kMany in `stopped`, and a pass back from wide_run: pack_skip.  Returns kMany where the next wave needs it again.
+// kMany in `stopped`, or from wide_run: pack_skip.  Returns kMany where the next wave needs it again.
 template <int NCH, class Job>
 __device__ __noinline__ unsigned pack_serve(Job job, PackLds* L, unsigned stopped, const int* abort_flag)
 {
     const int lane = __lane_id();
-    bool many = (stopped & kMany) != 0;
+    int many = (stopped & kMany) ? 1 : 0;
     for (int h = 0; h < 2; h++) {
         if (!((stopped >> h) & 1)) continue;
         PackSlot& S = L->slot[h];
         bool go = false;
         for (;;) {
             if (uni(S.phase) != PH_IDLE && uni(S.status) == LA_GROW) {
-                wide_run<NCH>(L, h, abort_flag);
+                many |= uni(wide_run<NCH>(L, h, abort_flag, many));
                 go = uni(S.running) != 0;
-                many |= go;
                 if (lane == 0) {
                     S.running = 0;
                     if (go) S.status = LA_OK;
