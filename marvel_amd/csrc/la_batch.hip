@@ -58,7 +58,7 @@ static size_t full_scratch_bytes(int ntasks, int maxlen, int tspace)
     size_t lv = 0;
     for (const Level& L : plan.lv)
         lv = std::max(lv, carve_bytes(kSlots * std::min(L.waves, ntasks), L.pool_cap, plan.pts_cap, plan.latr_cap));
-    return kCounterBytes + 2 * align_up((size_t)ntasks * sizeof(int)) + lv;
+    return kCounterBytes + 2 * align_up((size_t)ntasks * sizeof(int)) + lv + kCarveSlack;
 }
 
 static int device_batch_locked(BatchWorkspace* W, const MiAlignParams* prm, const uint64_t* d_packed,

@@ -272,6 +272,8 @@ constexpr int kSlots = 2;   // alignments a wave holds, each with its own scratc
 
 static const int kCounterBytes = 4096;   // 256 bytes of counters, then the length classes of a queue
 
+constexpr size_t kCarveSlack = 3 * 256;   // what a level's three pieces lose to their alignment, at most
+
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 static size_t wave_bytes(int pool_cap, int pts_cap, int latr_cap)
@@ -406,7 +408,7 @@ static int run_batch(DevSpec sp, const uint64_t* pk, const MiLaTask* tasks, int 
     int which = 0;
     for (int level = first; level < 4 && n > 0; level++) {
         const Level& L = plan.lv[level];
-        const size_t per = kSlots * wave_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap) + 3 * 256;
+        const size_t per = kSlots * wave_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap) + kCarveSlack;
         long long g = std::min<long long>(L.waves, n);
         const long long fit = (area.bytes - fixed) / per;
         if (g > fit) g = fit;

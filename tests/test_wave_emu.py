@@ -79,3 +79,18 @@ def test_trace_spacings_beyond_24_bits(emu, tspace):
 @pytest.mark.parametrize("tspace", [1, 2, 100, 2**23, 2**24])
 def test_a_read_of_more_than_2_to_23_bases(emu, tspace):
     assert check(emu, long_read_task(tspace)) == 1
+
+
+def wide_task(width, length=3000, tspace=100):
+    """One task that starts on `width` diagonals."""
+    ts = latasks.make_tasks(1, 7, lmin=length, lmax=length + 1, emin=0.05, emax=0.1, offmax=0, tspace=tspace)
+    par = ts.par.copy()
+    par[:, 3] -= width // 2
+    par[:, 4] = par[:, 3] + width - 1
+    return latasks.TaskSet(ts.ave_corr, ts.tspace, ts.freq, ts.reads, par)
+
+
+def test_a_single_task_beyond_the_widest_window(emu):
+    """The workspace of a batch of one holds the last level's scratch; the task keeps status 1 (window)."""
+    with emu_lib.in_place_of_gpu(emu):
+        assert la_batch(wide_task(1100))[1].tolist() == [1]
