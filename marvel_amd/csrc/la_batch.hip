@@ -56,8 +56,10 @@ static size_t full_scratch_bytes(int ntasks, int maxlen, int tspace)
 {
     const BatchPlan plan = make_plan(maxlen, tspace, mi_num_cus());
     size_t lv = 0;
-    for (const Level& L : plan.lv)
-        lv = std::max(lv, carve_bytes(kSlots * std::min(L.waves, ntasks), L.pool_cap, plan.pts_cap, plan.latr_cap));
+    for (const Level& L : plan.lv) {
+        const int slots = wave_slots(L, ntasks, INT64_MAX, mi_num_cus()) * std::min(L.waves, ntasks);
+        lv = std::max(lv, carve_bytes(slots, L.pool_cap, plan.pts_cap, plan.latr_cap));
+    }
     return kCounterBytes + 2 * align_up((size_t)ntasks * sizeof(int)) + lv + kCarveSlack;
 }
 

@@ -37,8 +37,9 @@ struct BatchScratch {
     int pool_cap;
     Peb* pts;
     int pts_cap;
-    uint16_t* latr;   // per wave: 4 * maxtp u16 (A and B traces, each with maxtp before and after its origin)
+    uint16_t* latr;   // per slot: 4 * maxtp u16 (A and B traces, each with maxtp before and after its origin)
     int latr_cap;
+    int slots;        // alignments a wave holds, each with a slot of scratch
 };
 
 // Arguments of a launch, read through the kernarg segment.
@@ -61,7 +62,7 @@ struct BatchArgs {
 };
 
 // The tasks of a launch as the packed aligner's job (la_pack.hpp): half h of
-// workgroup b owns scratch slot 2 b + h.
+// workgroup b owns scratch slot ws.slots b + h.
 // (NCH: each kernel has its own copy, so its registers fit that kernel's.)
 template <int NCH>
 struct BatchJob {
@@ -81,7 +82,7 @@ struct BatchJob {
         const int i = a->order ? uni(a->order[t]) : t;
         if (lane == 0) {
             const MiLaTask tk = a->tasks[i];
-            const int slot = 2 * blockIdx.x + h;
+            const int slot = a->ws.slots * blockIdx.x + h;
             const int TS = a->sp.tspace;
             const int maxtp = 2 * ((tk.alen > tk.blen ? tk.alen : tk.blen) / TS + 2);
             uint16_t* latr = a->ws.latr + (size_t)slot * a->ws.latr_cap;
@@ -166,8 +167,8 @@ struct BatchJob {
     }
 };
 
-// A persistent grid of single-wave workgroups.  With a wave for every task
-// the upper halves stay idle.
+// A persistent grid of single-wave workgroups; with one slot a wave the upper
+// halves stay idle.
 template <int NCH>
 __global__ __launch_bounds__(64, NCH == 2 ? kPackWaves : 1) void la_batch_kernel(BatchArgs)
 {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(64, NCH == 2 ? kPackWaves : 1) void la_batch_kernel
     sp.tspace = a->sp.tspace;
     sp.ave_path = a->sp.ave_path;
     pack_tables(L, sp);
-    pack_run<NCH>(L, BatchJob<NCH>{args, ti}, a->norder > (int)gridDim.x, a->abort_flag);
+    pack_run<NCH>(L, BatchJob<NCH>{args, ti}, a->ws.slots == 2, a->abort_flag);
 }
 
 // status of every task a launch covers := LA_UNRUN
@@ -268,7 +269,18 @@ struct Level {
     int waves;   // upper bound; the scratch may cap it
 };
 constexpr int kWideLevel = 2;   // the first level of kWideNch
-constexpr int kSlots = 2;   // alignments a wave holds, each with its own scratch
+
+// Alignments a wave holds at level L when n tasks run and the scratch has room
+// for `fit`.  One where every task gets a wave of its own, and where the
+// scratch leaves SIMDs without a wave: two alignments in lock step take longer
+// than one, so they are worth it only where waves share a SIMD.
+// (The 64 MiB of mi_la_batch_device_noalloc hold about 120: with two a wave
+// 4,000 tasks of 1 - 60 kb took 23.2 ms and 200,000 of 0.3 - 1 kb 220 ms, with
+// one 16.3 and 160 ms.)
+static int wave_slots(const Level& L, long long n, long long fit, int cus)
+{
+    return n > L.waves && fit > 4LL * cus ? 2 : 1;
+}
 
 static const int kCounterBytes = 4096;   // 256 bytes of counters, then the length classes of a queue
 
@@ -276,30 +288,31 @@ constexpr size_t kCarveSlack = 3 * 256;   // what a level's three pieces lose to
 
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-static size_t wave_bytes(int pool_cap, int pts_cap, int latr_cap)
+static size_t slot_bytes(int pool_cap, int pts_cap, int latr_cap)
 {
     return (size_t)pool_cap * sizeof(Peb) + (size_t)2 * pts_cap * sizeof(Peb) + (size_t)latr_cap * sizeof(uint16_t);
 }
 
-// carve `waves` slots of scratch at p (256-byte aligned pieces)
-static BatchScratch carve(char* p, int waves, int pool_cap, int pts_cap, int latr_cap)
+// carve n slots of scratch at p (256-byte aligned pieces)
+static BatchScratch carve(char* p, int n, int pool_cap, int pts_cap, int latr_cap)
 {
     BatchScratch s;
     s.pool_cap = pool_cap;
     s.pts_cap = pts_cap;
     s.latr_cap = latr_cap;
     s.pools = (Peb*)p;
-    p += align_up((size_t)waves * pool_cap * sizeof(Peb));
+    p += align_up((size_t)n * pool_cap * sizeof(Peb));
     s.pts = (Peb*)p;
-    p += align_up((size_t)waves * 2 * pts_cap * sizeof(Peb));
+    p += align_up((size_t)n * 2 * pts_cap * sizeof(Peb));
     s.latr = (uint16_t*)p;
+    s.slots = 1;
     return s;
 }
 
-static size_t carve_bytes(int waves, int pool_cap, int pts_cap, int latr_cap)
+static size_t carve_bytes(int n, int pool_cap, int pts_cap, int latr_cap)
 {
-    return align_up((size_t)waves * pool_cap * sizeof(Peb)) + align_up((size_t)waves * 2 * pts_cap * sizeof(Peb)) +
-           align_up((size_t)waves * latr_cap * sizeof(uint16_t));
+    return align_up((size_t)n * pool_cap * sizeof(Peb)) + align_up((size_t)n * 2 * pts_cap * sizeof(Peb)) +
+           align_up((size_t)n * latr_cap * sizeof(uint16_t));
 }
 
 static int launch_level(int nch, int grid, const MiLaTask* tasks, const int* order, int n, const uint64_t* pk,
@@ -408,16 +421,16 @@ static int run_batch(DevSpec sp, const uint64_t* pk, const MiLaTask* tasks, int 
     int which = 0;
     for (int level = first; level < 4 && n > 0; level++) {
         const Level& L = plan.lv[level];
-        const size_t per = kSlots * wave_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap) + kCarveSlack;
-        long long g = std::min<long long>(L.waves, n);
-        const long long fit = (area.bytes - fixed) / per;
-        if (g > fit) g = fit;
-        while (g > 0 && carve_bytes(kSlots * (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap) > area.bytes - fixed) g--;
+        const size_t slot = slot_bytes(L.pool_cap, plan.pts_cap, plan.latr_cap), room = area.bytes - fixed;
+        const long long fit = room > kCarveSlack ? (long long)((room - kCarveSlack) / slot) : 0;
+        const int slots = wave_slots(L, n, fit, mi_num_cus());
+        const long long g = std::min<long long>(std::min<long long>(L.waves, n), fit / slots);
         if (g <= 0) {
             mi_set_error("batch: scratch too small for one wave of this level");
             return MI_ERR_ARG;
         }
-        const BatchScratch ws = carve(area.base + fixed, kSlots * (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap);
+        BatchScratch ws = carve(area.base + fixed, slots * (int)g, L.pool_cap, plan.pts_cap, plan.latr_cap);
+        ws.slots = slots;
         int* retry = lists[which];
         if (level == first && cur == nullptr && n > g) {
             // (the second list is free until the next level's retries)

@@ -2,6 +2,7 @@
 oracle: the kernels of marvel_amd/csrc/la_pack.hpp and la_batch_core.hpp
 compiled by g++, one fiber per lane."""
 
+import ctypes as C
 import os
 import shutil
 
@@ -14,6 +15,7 @@ import oracle_lib
 import repeat_tasks
 from marvel_amd import latasks
 from marvel_amd.align import la_batch
+from marvel_amd.lib import MiLaResult, MiLaTask, MiTuning, params
 from repeat_tasks import long_read_task
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None or os.uname().machine != "x86_64",
@@ -22,10 +24,13 @@ pytestmark = pytest.mark.skipif(shutil.which("g++") is None or os.uname().machin
 
 @pytest.fixture(scope="module", params=[False, True], ids=["", "garbage"])
 def emu(request):
-    """One library as built, one whose LDS holds garbage when a kernel starts."""
-    os.environ.setdefault("MI_EMU_CUS", "1")
+    """One library as built, one whose LDS holds garbage when a kernel starts.
+    On one CU with 4 waves, so that batches of more than 4 tasks use both halves of a wave."""
+    os.environ["MI_EMU_CUS"] = "1"
     emu_lib.build()
-    return emu_lib.Lib(request.param)
+    lib = emu_lib.Lib(request.param)
+    assert lib.mi_set_tuning(C.byref(MiTuning(0, 0, 0, 4, 0))) == 0
+    return lib
 
 
 def check(emu, ts):
@@ -94,3 +99,43 @@ def test_a_single_task_beyond_the_widest_window(emu):
     """The workspace of a batch of one holds the last level's scratch; the task keeps status 1 (window)."""
     with emu_lib.in_place_of_gpu(emu):
         assert la_batch(wide_task(1100))[1].tolist() == [1]
+
+
+def noalloc(emu, ts):
+    """mi_la_batch_device_noalloc over a TaskSet (device memory is host memory here): (rc, status, results, traces)."""
+    words, aw, bw = ts.packed()
+    tasks, res = (MiLaTask * ts.n)(), (MiLaResult * ts.n)()
+    for i in range(ts.n):
+        t = tasks[i]
+        t.aword, t.bword = int(aw[i]), int(bw[i])
+        t.alen, t.blen, t.comp, t.low, t.hgh, t.anti, t.lbord, t.hbord = (int(x) for x in ts.par[i])
+    cap = int(sum(4 * (max(int(p[0]), int(p[1])) // ts.tspace + 2) for p in ts.par)) + 16
+    tr, used = np.zeros(cap, dtype=np.uint16), C.c_ulonglong(0)
+    prm = params(ts.ave_corr, ts.tspace, ts.freq)
+    rc = emu.mi_la_batch_device_noalloc(C.byref(prm), words.ctypes.data, words.shape[0], tasks, ts.n, res,
+                                        tr.ctypes.data, cap, C.byref(used))
+    out = [((r.abpos, r.bbpos, r.aepos, r.bepos, r.diffs, r.atlen, r.b_abpos, r.b_bbpos, r.b_aepos, r.b_bepos, r.diffs,
+             r.btlen), tr[r.atrace:r.atrace + r.atlen], tr[r.btrace:r.btrace + r.btlen]) for r in res]
+    return rc, np.array([r.status for r in res]), out
+
+
+@pytest.mark.parametrize("n", [1, 130])
+def test_fixed_scratch_batch(emu, n):
+    """130: more tasks than the 64 MiB hold waves."""
+    ts = latasks.make_tasks(n, 12, lmin=200, lmax=400, emin=0.05, emax=0.2, offmax=10)
+    want, st = oracle_lib.run_tasks(ts)
+    rc, status, got = noalloc(emu, ts)
+    keep = [i for i in range(n) if st[i] == 0]
+    assert rc == 0 and len(keep) > 0.9 * n
+    assert not la_golden.diff([got[i] for i in keep], [want[i] for i in keep], status[keep])
+
+
+def test_fixed_scratch_holds_one_wave_of_the_last_level(emu):
+    """A read of 500,000 bases at a spacing of 1: the last level's pool, chain
+    points and traces fit into 64 MiB once, not twice."""
+    ts = wide_task(1100, tspace=1)
+    long = np.concatenate([ts.reads[0], np.zeros(500_000 - len(ts.reads[0]), dtype=np.uint8)])
+    par = ts.par.copy()
+    par[0, 0] = len(long)
+    rc, status, _ = noalloc(emu, latasks.TaskSet(ts.ave_corr, 1, ts.freq, [long, ts.reads[1]], par))
+    assert rc == 0 and status.tolist() == [1]
