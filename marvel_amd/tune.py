@@ -3,10 +3,12 @@
 The report kernel's waves per CU at its first and its 256-diagonal window,
 the pebble pool of the first window and the batched aligner's waves per CU at
 its first and its 256-diagonal window (MiTuning, include/marvl_align.h)
-change how fast a pass runs, never what it writes.  The tuner times short calibration runs of the caller's own
-workload with each candidate, keeps the fastest, and stores the choice per
-device (architecture and compute units) in a JSON cache, so later processes
-on the same kind of GPU load it instead of calibrating again.
+change how fast a pass runs, never what it writes.  The tuner times short
+calibration runs of the caller's own workload with each candidate, keeps the
+fastest, or the default where none is faster by more than the runs differ, and
+stores the choice per device (architecture and compute units) and kernel
+generation in a JSON cache, so later processes on the same kind of GPU load it
+instead of calibrating again.
 
     python -m marvel_amd.tune --show        # the cached choice for this GPU
 """
@@ -14,6 +16,7 @@ on the same kind of GPU load it instead of calibrating again.
 from __future__ import annotations
 
 import ctypes as C
+import hashlib
 import json
 import os
 import time
@@ -29,6 +32,11 @@ L1_CANDIDATES = (4, 8, 12)
 # (first window, 256-diagonal window): the levels are timed apart, so each
 # run scores one candidate of each and the two are chosen independently
 BATCH_CANDIDATES = ((16, 2), (20, 4), (24, 8))
+# a candidate replaces the default when it is faster by more than this share
+# (two runs of one shape differ by 1 to 3 %)
+MARGIN = 0.03
+# raised when the kernels change what the fields mean (2: two alignments per wave)
+GENERATION = 2
 
 
 def cache_path() -> str:
@@ -43,6 +51,20 @@ def device_key() -> str:
     if lib.mi_device_info(name, 64, C.byref(cus)) != 0:
         raise RuntimeError(lib.last_error())
     return f"{name.value.decode()}:{cus.value}cu"
+
+
+def cache_key() -> str:
+    """The device and the kernels that a stored choice holds for."""
+    shapes = repr((GENERATION, FIELDS, sorted(DEFAULT.items()), REPORT_CANDIDATES, L1_CANDIDATES, BATCH_CANDIDATES))
+    return f"{device_key()}:{hashlib.sha256(shapes.encode()).hexdigest()[:8]}"
+
+
+def pick(times: dict, default):
+    """The fastest of `times` (seconds per candidate), or the default where
+    none is faster by more than MARGIN -- a level that no task of the
+    calibration reaches reads 0 for every candidate."""
+    best = min(times, key=times.get)
+    return best if times[best] < (1 - MARGIN) * times[default] else default
 
 
 def apply(choice: dict):
@@ -60,7 +82,7 @@ def current() -> dict:
 def load_cached() -> dict | None:
     try:
         with open(cache_path()) as f:
-            return json.load(f).get(device_key())
+            return json.load(f).get(cache_key())
     except (OSError, ValueError):
         return None
 
@@ -73,7 +95,7 @@ def save(choice: dict):
             allc = json.load(f)
     except (OSError, ValueError):
         allc = {}
-    allc[device_key()] = choice
+    allc[cache_key()] = choice
     tmp = p + ".tmp"
     with open(tmp, "w") as f:
         json.dump(allc, f, indent=1, sort_keys=True)
@@ -121,13 +143,15 @@ def tune_report(step) -> dict:
         for w, p in REPORT_CANDIDATES:
             apply({**base, "report_waves_per_cu": w, "report_pool_log2": p})
             timings[f"w{w}_p{p}"] = _time_report(step)
-    w, p = min(REPORT_CANDIDATES, key=lambda c: timings[f"w{c[0]}_p{c[1]}"])
+    w, p = pick({c: timings[f"w{c[0]}_p{c[1]}"] for c in REPORT_CANDIDATES},
+                (DEFAULT["report_waves_per_cu"], DEFAULT["report_pool_log2"]))
     best = {**base, "report_waves_per_cu": w, "report_pool_log2": p}
     with _FirstLevel(1):
         for l1 in L1_CANDIDATES:
             apply({**best, "report_l1_waves_per_cu": l1})
             timings[f"l1_{l1}"] = _time_report(step)
-    best["report_l1_waves_per_cu"] = min(L1_CANDIDATES, key=lambda c: timings[f"l1_{c}"])
+    best["report_l1_waves_per_cu"] = pick({c: timings[f"l1_{c}"] for c in L1_CANDIDATES},
+                                          DEFAULT["report_l1_waves_per_cu"])
     apply(best)
     return {"choice": best, "timings_s": {k: round(v, 5) for k, v in timings.items()}}
 
@@ -145,7 +169,8 @@ def tune_batch(run) -> dict:
         work = run()
         narrow[w0] = min(narrow.get(w0, float("inf")), work[2] / 1e6)
         wide[w1] = sum(work[3:6]) / 1e6
-    best = {**base, "batch_waves_per_cu": min(narrow, key=narrow.get), "batch_wide_waves_per_cu": min(wide, key=wide.get)}
+    best = {**base, "batch_waves_per_cu": pick(narrow, DEFAULT["batch_waves_per_cu"]),
+            "batch_wide_waves_per_cu": pick(wide, DEFAULT["batch_wide_waves_per_cu"])}
     apply(best)
     timings = {**{f"b{k}": v for k, v in narrow.items()}, **{f"wide{k}": v for k, v in wide.items()}}
     return {"choice": best, "timings_s": {k: round(v, 5) for k, v in timings.items()}}
