@@ -165,12 +165,12 @@ def test_output_arena_overflow_reruns(tmp_path, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("level", [1, 2, 3, 4])
+@pytest.mark.parametrize("level", [0, 1, 2, 3])
 def test_every_report_window_matches_reference(tmp_path, monkeypatch, level):
-    """Every pair started at aligner window level 1-4 (128 / 256 / 1,024
-    diagonals, then the large pools and arenas) writes the reference's .las:
-    the wide report kernels, otherwise run only for the few pairs that
-    outgrow the 64-lane window, on a whole workload."""
+    """Every pair started at report level 0-3 (windows of 128, 256 and 1,024
+    diagonals, then 1,024 with the large pools and arenas) writes the
+    reference's .las: the wider report kernels, otherwise run only for the
+    few pairs that outgrow 128 diagonals, on a whole workload."""
     from marvel_amd.daligner import Daligner
 
     case = "rep_j8"
