@@ -303,8 +303,9 @@ const char *mi_last_error(void);
 int mi_device_count(void);
 
 /* Device self-tests of the wave64 building blocks (0: persistent task loop,
- * 1: lane scans / shuffles / ballots, 2: 2-bit snake matcher); the caller
- * checks `out` against its own CPU computation. */
+ * 1: lane scans / shuffles / ballots, 2: the trace kernel's 2-bit matchers,
+ * 3: the aligner's lane moves, 4: its 2-bit snake, 5: its path columns); the
+ * caller checks `out` against its own CPU computation. */
 int mi_selftest(int which, const void *in, long long nin, const void *in2, long long nin2, const void *q, int nq,
                 int arg, void *out, long long nout);
 

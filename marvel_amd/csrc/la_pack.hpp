@@ -303,14 +303,14 @@ __device__ __forceinline__ int snake_len(SeqWord* A, SeqWord* B, int m, int x, i
 
 // The last 61 columns of a path as mismatch bits, latest at bit 3, with bit 2
 // set (the mismatch column every step begins with): one more mismatch and s
-// matches.  m: matches among the last 60.
+// matches.  m: matches among them.
 __device__ __forceinline__ void add_columns(uint64_t& N, int& m, int s)
 {
     const int sc = min(s, 61);
     m += __popcll(N >> (63 - sc)) - 1;
     N = (N << (sc + 1)) | 4;
 }
-constexpr uint64_t kColsInit = (1ull << 63) | 4;   // 60 matches
+constexpr uint64_t kColsInit = (1ull << 63) | 4;   // a mismatch, then 60 matches
 
 // the smallest score of a suffix of the last 30 columns; >= 0: the path may be trimmed here (TABLE and SCORE of
 // dalign/align.c:884-896)

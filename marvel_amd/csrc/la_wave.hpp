@@ -85,7 +85,6 @@ __device__ __forceinline__ int match_rev(const uint64_t* A, const uint64_t* B, i
 }
 
 // ---- cross-lane helpers ----------------------------------------------------
-__device__ __forceinline__ int shfl_i(int v, int src) { return __shfl(v, src, 64); }
 __device__ __forceinline__ int rdl(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ uint64_t rdl64(uint64_t v, int lane)
 {

@@ -1,10 +1,11 @@
-// Device self-tests of the wave64 building blocks the aligner relies on
-// (cross-lane scans, neighbour gathers, ballots/mbcnt, the 2-bit snake
-// matcher, the persistent task loop).  Each test writes plain per-lane /
+// Device self-tests of the wave64 building blocks the aligner and the trace
+// kernel rely on (cross-lane scans, neighbour gathers, ballots/mbcnt, the 2-bit
+// matchers, a path's columns, the persistent task loop), called as the kernels
+// call them.  Each test writes plain per-lane /
 // per-task outputs that the host checks against a CPU computation.
 #include <hip/hip_runtime.h>
 
-#include "la_wave.hpp"
+#include "la_pack.hpp"
 #include "mi_common.h"
 
 namespace mi {
@@ -43,8 +44,8 @@ __global__ __launch_bounds__(64) void st_lanes(const int* in, int thr, int* out)
     }
     int exc2 = __shfl_up(inc2, 1, 64);
     if (lane == 0) exc2 = INT32_MAX;
-    const int up = shfl_i(v, (lane + 63) & 63);
-    const int dn = shfl_i(v, (lane + 1) & 63);
+    const int up = __shfl(v, (lane + 63) & 63, 64);
+    const int dn = __shfl(v, (lane + 1) & 63, 64);
     const unsigned long long odd = __ballot(v & 1);
     int rl = -7;
     if (odd) rl = rdl(v, lowest_lane(odd));
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(64) void st_lanes(const int* in, int thr, int* out)
     o[0] = excl; o[1] = exc2; o[2] = up; o[3] = dn; o[4] = rl; o[5] = rank; o[6] = any; o[7] = __popcll(odd);
 }
 
-// test 2: snake matcher; per lane one query (x, y, lim, dir) on packed A/B
+// test 2: the trace kernel's matchers; per lane one query (x, y, lim, dir) on packed A/B
 __global__ __launch_bounds__(64) void st_match(const uint64_t* A, const uint64_t* B, const int* q, int n, int* out)
 {
     const int i = blockIdx.x * 64 + __lane_id();
@@ -66,92 +67,57 @@ __global__ __launch_bounds__(64) void st_match(const uint64_t* A, const uint64_t
     out[2 * i + 1] = mism ? 1 : 0;
 }
 
-// value of lane (L-1) & 63 / (L+1) & 63: DPP wave_ror:1 / wave_rol:1, full-rate
-// VALU moves (no LDS traffic).  All 64 lanes must be active.
-// (every lane has a source, so no "old" value is needed: one v_mov_b32_dpp)
-__device__ __forceinline__ int lane_below(int v) { return __builtin_amdgcn_mov_dpp(v, 0x13C, 0xF, 0xF, false); }
-__device__ __forceinline__ int lane_above(int v) { return __builtin_amdgcn_mov_dpp(v, 0x134, 0xF, 0xF, false); }
-// Wave-wide scans from DPP row moves (no LDS): row_shl:n / row_shr:n read
-// lane L+n / L-n of the same 16-lane row, row_bcast:15 / :31 hand the last
-// lane of a row (of two rows) to the next row(s).  Lanes without a source
-// read 0 (bound_ctrl), the identity of max over non-negative values, so each
-// level is a single v_max_i32 with a DPP operand.
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ int dpp0(int v)
-{
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xF, true);
-}
-// inclusive max over lanes >= L of x >= 0
-__device__ __forceinline__ int suffix_max_nn(int x)
-{
-    x = max(x, dpp0<0x101>(x));   // row_shl:1
-    x = max(x, dpp0<0x102>(x));   // row_shl:2
-    x = max(x, dpp0<0x104>(x));   // row_shl:4
-    x = max(x, dpp0<0x108>(x));   // row_shl:8
-    // lane 16r now holds row r's maximum; lanes of row r add the rows above
-    // it, selected with arithmetic masks (-1 / 0) rather than lane masks
-    const int s1 = __builtin_amdgcn_readlane(x, 16), s2 = __builtin_amdgcn_readlane(x, 32);
-    const int s3 = __builtin_amdgcn_readlane(x, 48);
-    int row = __lane_id() >> 4;
-    asm volatile("" : "+v"(row));   // keeps the row masks from being hoisted into (spilled) SGPR lane masks
-    const int m1 = (row - 1) >> 31, m2 = (row - 2) >> 31, m3 = (row - 3) >> 31;
-    return max(max(x, s1 & m1), max(s2 & m2, s3 & m3));
-}
-// inclusive max over lanes <= L of x >= 0
-__device__ __forceinline__ int prefix_max_nn(int x)
-{
-    x = max(x, dpp0<0x111>(x));        // row_shr:1
-    x = max(x, dpp0<0x112>(x));        // row_shr:2
-    x = max(x, dpp0<0x114>(x));        // row_shr:4
-    x = max(x, dpp0<0x118>(x));        // row_shr:8
-    x = max(x, dpp0<0x142, 0xA>(x));   // row_bcast:15 into rows 1, 3
-    x = max(x, dpp0<0x143, 0xC>(x));   // row_bcast:31 into rows 2, 3
-    return x;
-}
-// value of lane L+1 / L-1; the lane without one (63 / 0) gets `edge`
-// (DPP wave_shl:1 / wave_shr:1)
-__device__ __forceinline__ int lane_above_or(int v, int edge) { return __builtin_amdgcn_update_dpp(edge, v, 0x130, 0xF, 0xF, false); }
-__device__ __forceinline__ int lane_below_or(int v, int edge) { return __builtin_amdgcn_update_dpp(edge, v, 0x138, 0xF, 0xF, false); }
-// inclusive max over lanes >= L (x >= -1).  GATHER: the lanes reversed by one
-// ds_bpermute each way around the DPP prefix scan, for passes that run many
-// waves per SIMD (the LDS pipe is idle there, the VALU is not); otherwise
-// the DPP suffix scan, which keeps the two LDS round trips off the path of a
-// wave that runs alone (the wider windows).
-template <bool GATHER>
-__device__ __forceinline__ int wave_suffix_max(int x)
-{
-    if constexpr (GATHER) {
-        const int r = 63 - __lane_id();
-        return __shfl(prefix_max_nn(__shfl(x + 1, r, 64)), r, 64) - 1;
-    } else {
-        return suffix_max_nn(x + 1) - 1;
-    }
-}
-// inclusive min over lanes <= L (any x): the max of INT32_MAX - x >= 0
-__device__ __forceinline__ int wave_prefix_min(int x) { return 2147483647 - prefix_max_nn(2147483647 - x); }
-
-// fields of lane L + sel (sel in {-1, 0, +1}, wrapping like (L + sel) & 63)
-__device__ __forceinline__ int pick3(int v, int sel)
-{
-    const int b = lane_below(v), a = lane_above(v);
-    return sel < 0 ? b : (sel > 0 ? a : v);
-}
-// test 3: DPP lane moves; per lane: [lane_below(v), lane_above(v), the
-// scans, the edge moves, the DPP suffix max, pick3 with sel = L % 3 - 1]
-__global__ __launch_bounds__(64) void st_dpp(const int* in, int* out)
+// test 3: the packed aligner's lane moves (la_pack.hpp); per lane: the inclusive prefix maxima of its half and of the
+// wave, the values of lanes L - 1 and L + 1 (twice, the second time with the sentinel at the wave's ends), two
+// gathers, and what it sees of the ballot of v's lowest bit
+constexpr int kMoves = 13;
+__global__ __launch_bounds__(64) void st_moves(const int* in, int* out)
 {
     const int lane = __lane_id();
     const int v = in[blockIdx.x * 64 + lane];
-    int* o = out + (blockIdx.x * 64 + lane) * 8;
-    o[0] = lane_below(v);
-    o[1] = lane_above(v);
-    // the aligner's scans: suffix max over values >= -1, prefix min over values >= 0
-    o[2] = wave_suffix_max<true>(v);
-    o[3] = wave_prefix_min(v < 0 ? 2147483647 : v);
-    o[4] = lane_above_or(v, -7);
-    o[5] = lane_below_or(v, -9);
-    o[6] = wave_suffix_max<false>(v);
-    o[7] = pick3(v, lane % 3 - 1);
+    int* o = out + (blockIdx.x * 64 + lane) * kMoves;
+    o[0] = prefix_max<false>(v);
+    o[1] = prefix_max<true>(v);
+    o[2] = dpp_shr1(v);
+    o[3] = dpp_shl1(v);
+    o[4] = from_below(v);
+    o[5] = from_above(v);
+    o[6] = bperm(v, (7 * lane + 3) & 63);
+    const uint64_t w = bperm64(((uint64_t)(uint32_t)v << 32) | (uint32_t)~v, lane ^ 33);
+    o[7] = (int)(w >> 32);
+    o[8] = (int)w;
+    const unsigned long long odd = ballot(v & 1);
+    const uint32_t h = hmask(-(lane >> 5), odd);
+    o[9] = lane_in(odd) ? 1 : 0;
+    o[10] = (int)h;
+    o[11] = h ? top_bit(h) : -1;
+    o[12] = h ? low_bit(h) : -1;
+}
+
+// test 4: snake_len; per lane one query (x, y, lim, m), x and y in the pass's direction
+__global__ __launch_bounds__(64) void st_snake(const uint64_t* A, const uint64_t* B, const int* q, int n, int* out)
+{
+    const int i = blockIdx.x * 64 + __lane_id();
+    const bool in = i < n;   // every lane takes part
+    const int x = in ? q[4 * i] : 0, y = in ? q[4 * i + 1] : 0, lim = in ? q[4 * i + 2] : 0, m = in ? q[4 * i + 3] : 0;
+    const int s = snake_len((SeqWord*)A, (SeqWord*)B, m, x, y, lim, lim > 0);
+    if (in) out[i] = s;
+}
+
+// test 5: a path's columns; per lane `steps` snake lengths, after each of them the matches among the last 61 columns
+// and the smallest score of a suffix of the last 30
+__global__ __launch_bounds__(64) void st_columns(DevSpec sp, const int* in, int steps, int* out)
+{
+    __shared__ PackLds L;
+    pack_tables(L, sp);
+    const int i = blockIdx.x * 64 + __lane_id();
+    uint64_t N = kColsInit;
+    int m = kPathLen;
+    for (int t = 0; t < steps; t++) {
+        add_columns(N, m, in[i * steps + t]);
+        out[2 * (i * steps + t)] = m;
+        out[2 * (i * steps + t) + 1] = min_suffix(L, L.w_match, L.w_all, N);
+    }
 }
 
 }  // namespace mi
@@ -183,8 +149,23 @@ extern "C" int mi_selftest(int which, const void* in, long long nin, const void*
                                          (int*)dout);
         break;
     case 3:
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(st_dpp), dim3((int)(nin / 256)), dim3(64), 0, 0, (const int*)din, (int*)dout);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(st_moves), dim3((int)(nin / 256)), dim3(64), 0, 0, (const int*)din, (int*)dout);
         break;
+    case 4:
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(st_snake), dim3((nq + 63) / 64), dim3(64), 0, 0, (const uint64_t*)din + 1,
+                           (const uint64_t*)din2 + 1, (const int*)dq, nq, (int*)dout);
+        break;
+    case 5: {
+        MiAlignParams prm = {};
+        prm.ave_corr = 0.70;
+        prm.trace_space = 100;
+        for (float& f : prm.freq) f = 0.25f;
+        const DevSpecHost* ds = mi_spec_device(&prm);
+        if (ds == nullptr) goto done;
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(st_columns), dim3((int)(nin / (256LL * arg))), dim3(64), 0, 0, ds->spec,
+                           (const int*)din, arg, (int*)dout);
+        break;
+    }
     default:
         rc = MI_ERR_ARG;
         goto done;
