@@ -37,21 +37,22 @@
 //   * What only changes at events lives in LDS, written by the lane that owns
 //     the event: the trim point, the best point's y, the boundary point.
 //
-// What bounds it, on a full GPU: VALU issue -- 2.59e10 wave64 VALU
-// instructions per report launch on the 5 Mbp / 30x block (190 per step of two
-// alignments), 42 ms of the 53 ms it takes at one per SIMD every 4 cycles; one
+// What bounds it, on a full GPU: VALU issue -- 2.66e10 wave64 VALU
+// instructions per report launch on the 5 Mbp / 30x block (196 per step of two
+// alignments), 43 ms of the 45 ms it takes at one per SIMD every 4 cycles; one
 // alignment per wave needed 5.2e10 and 96 ms (and 6.6 ms more for the pairs
 // wider than 64 diagonals, run again at 128).  So the sets of lanes are kept as
 // the compares' own masks (ballot, lane_in: an integer made of a condition and
-// compared again took 2 instructions more each, 64 ms a launch), products are
-// 24-bit, and the reads and the pool are addressed as HBM (a flat access also
-// holds up every wait for LDS).  Where few alignments are left (repeat-rich
+// compared again takes 2 instructions more each), products are 24-bit, and the
+// reads and the pool are addressed as HBM (a flat access also holds up every
+// wait for LDS).  Where few alignments are left (repeat-rich
 // blocks: one pair with 90 alignments one after another, 55 % of the CUs busy
 // over the launch) it is the latency of one wave's step, about 1.5 us.
-// Waves per SIMD: 4, 5, 6 and 7 take 190, 178, 175, 179 ms a pass on the 5 Mbp
-// block and 66, 74, 56, 56 ms on 400,000 tasks that start off their diagonal;
-// repeat-rich blocks prefer fewer (214, 212, 217, 218 ms).  7 spills in the
-// loop, so 6.
+// Waves per SIMD, ms a pass against 6 in turn on one box:
+//   4: 5 Mbp block 186 : 179, repeat-rich 201 : 207, 400,000 tasks that start
+//      off their diagonal 54.2 : 48.4, 20,000 tasks 19.2 : 21.8
+//   5: 197 : 189, 254 : 259, 50.6 : 49.1, 19.8 : 21.6
+//   7: 177 : 174, 223 : 213, 47.6 : 48.0, 20.5 : 20.7 (spills in the loop)
 //
 // Persistent kernels: `Job` (a few pointers, passed by value) hands out
 // alignments (next) and takes their results (done); PackSlot says what it
@@ -120,6 +121,7 @@ struct PackLds {
     PackHot hot[2];
     int16_t suf[1 << kSufBits];   // smallest suffix sum of 10 columns given by their mismatches
     int w_all, w_match;           // score of a column: w_match for a match, w_match - w_all for a mismatch
+    int many;                     // the last wave of a pass passed many trace points (see skip_points)
     DevSpec sp;
     PackSlot slot[2];
     PackBand band[2];
@@ -218,8 +220,9 @@ __device__ __forceinline__ int hsel(int hm, int lo, int hi)
 // Wave priority (0..3) by the place in the queue: the queues hold the longest
 // alignments first, and a launch ends when the longest chain of waves does,
 // so the waves that hold it issue before the others of their SIMD.
-// (A 4 Mbp block 13.3 -> 11.7 ms a pass, 400,000 tasks 50.2 -> 46.7 ms; blocks
-// whose heavy pairs their seeds do not tell, 246.9 and 249.6 ms.)
+// (Without and with: 400,000 tasks 50.6 and 48.1 ms, 20,000 tasks 21.8 and
+// 21.5, 4 Mbp block 11.9 and 11.7, 5 Mbp block 179 and 178; repeat-rich block,
+// whose heavy pairs their seeds do not tell, 219 and 221.)
 __device__ __forceinline__ int queue_priority(int t, int n)
 {
     return t < n / 256 ? 3 : t < n / 32 ? 2 : t < n / 8 ? 1 : 0;
@@ -267,9 +270,9 @@ __device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_updat
 // forward, -1 reverse; x and y in the pass's coordinates), on the lanes where
 // `in` holds; every lane takes part.  32 bases a step: a second step is a
 // round trip to memory for the whole wave, and with 16 bases one of its lanes
-// asked for it in 9 of 10 steps at 16 % pair error (in 1 of 8 at 28 %).
-// (repeat-rich block 246.9 -> 242.3 ms a pass, long reads 235.1 -> 230.4 ms,
-// 64 tasks 3.27 -> 3.18 ms; the 28 % block 176.5 and 178.1 ms.)
+// asks for it in 9 of 10 steps at 16 % pair error (in 1 of 8 at 28 %).
+// (16 and 32 bases: 20,000 tasks 22.4 and 21.5 ms; 400,000 tasks, the 5 Mbp
+// and the repeat-rich block the same.)
 typedef Glob<const uint32_t> SeqWord;
 // the 32-base windows at x and y compared: bit pair i differs where base i does
 __device__ __forceinline__ uint64_t seq_diff(SeqWord* A, SeqWord* B, int m, int x, int y)
@@ -332,6 +335,7 @@ __device__ __forceinline__ void pack_tables(PackLds& L, const DevSpec& sp)
         L.sp = sp;
         L.w_match = all / 15;
         L.w_all = (all - none) / 15;
+        L.many = 0;
     }
     // both halves idle: the loop reads every field of a slot, also of one that never gets an alignment
     int* z = (int*)L.slot;
@@ -362,10 +366,11 @@ __device__ __forceinline__ void pack_tables(PackLds& L, const DevSpec& sp)
 // through a tandem repeat in one wave, the diagonal itself stays.  So only a
 // wave after one that passed kManyPoints points looks at the paths that end
 // that many points beyond t (a pebble lies on its path), and reads the marks of
-// their pebbles.  (Looking in every wave that crosses trace points cost 2.7 %
-// on the 5 Mbp block, 172.9 -> 177.7 ms a pass.)
+// their pebbles: pack_skip between two waves of the halves' loop, wide_run
+// instead of the numbers.  (Looking in every wave that crosses trace points
+// cost 2.7 % on the 5 Mbp block, 172.9 -> 177.7 ms a pass.)
 constexpr int kManyPoints = 120;
-constexpr unsigned kMany = 4;          // beside the halves to serve: the last wave passed many points
+constexpr unsigned kMany = 4;          // beside the halves to serve: `many` is set
 __device__ __forceinline__ int many_points(int TS) { return TS <= INT32_MAX / kManyPoints ? kManyPoints * TS : INT32_MAX; }
 // The first point from t on that lies beyond pebble h (point n lies at n TS + off): no point before it needs a pebble.
 __device__ __forceinline__ int skip_points(const Glob<Int4>* pool, int h, int t, int TS, int off, int m)
@@ -382,15 +387,13 @@ __device__ __forceinline__ int skip_points(const Glob<Int4>* pool, int h, int t,
 // their wave's trace points and records) or it ends (running = 0, status).
 // slot.dif < 0: the pass begins here, a forward pass from more diagonals than
 // a half holds.
-// many: whether the wave before the first passed many trace points; returned
-// for the wave before the one the pass goes on with.
 // Index i of the window (lane i & 63 of chunk i >> 6) holds diagonal kt - i.
 template <int NCH>
-__device__ __noinline__ int wide_run(PackLds* L, int h, const int* abort_flag, int many)
+__device__ __noinline__ void wide_run(PackLds* L, int h, const int* abort_flag)
 {
     constexpr int W = 64 * NCH;
     const int lane = __lane_id();
-    many = uni(many);
+    int many = uni(L->many);
     PackSlot& S = L->slot[h];
     PackHot& H = L->hot[h];
     PackBand& D = L->band[h];
@@ -719,33 +722,17 @@ __device__ __noinline__ int wide_run(PackLds* L, int h, const int* abort_flag, i
                 many = n >= kManyPoints ? 1 : 0;
                 break;
             }
-            if (many) {   // (see skip_points)
-                const int far = many_points(TS);
-                bool fA[NCH], fB[NCH], f = false;
-#pragma unroll
-                for (int j = 0; j < NCH; j++) {
-                    fA[j] = wA[j] && y[j] + kt - (64 * j + lane) - point_at<NCH>(tA[j], TS) >= far;
-                    fB[j] = wB[j] && y[j] - point_at<NCH>(tB[j], TS) - offB >= far;
-                    f |= fA[j] | fB[j];
-                }
-                many = 0;
-                if (any_lane(f)) {
-                    wave_sync();   // pebbles of this wave's other lanes
-#pragma unroll
-                    for (int j = 0; j < NCH; j++) {
-                        if (fA[j]) tA[j] = skip_points(pool, HA[j], tA[j], TS, 0, m);
-                        if (fB[j]) tB[j] = skip_points(pool, HB[j], tB[j], TS, offB, m);
-                    }
-                    n = kManyPoints;
-                    continue;
-                }
-            }
+            if (many) wave_sync();   // pebbles of this wave's other lanes
 #pragma unroll
             for (int j = 0; j < NCH; j++) {
                 if (!live(j)) continue;
                 const int k = kt - (64 * j + lane);
-                const bool pA = wA[j] && (dif == 0 || (int)(((unsigned)tA[j] << 24) - ((unsigned)HA[j] & ~(unsigned)kPebIdx)) > 0);
-                const bool pB = wB[j] && (dif == 0 || (int)(((unsigned)tB[j] << 24) - ((unsigned)HB[j] & ~(unsigned)kPebIdx)) > 0);
+                bool pA = wA[j] && (dif == 0 || (int)(((unsigned)tA[j] << 24) - ((unsigned)HA[j] & ~(unsigned)kPebIdx)) > 0);
+                bool pB = wB[j] && (dif == 0 || (int)(((unsigned)tB[j] << 24) - ((unsigned)HB[j] & ~(unsigned)kPebIdx)) > 0);
+                if (many) {   // (see skip_points; the marks themselves)
+                    if (wA[j]) pA = dif == 0 || ((pool[HA[j] & kPebIdx][3] ^ m) - m) < point_at<NCH>(tA[j], TS);
+                    if (wB[j]) pB = dif == 0 || ((pool[HB[j] & kPebIdx][3] ^ m) - m) < point_at<NCH>(tB[j], TS) + offB;
+                }
                 const unsigned long long ba = ballot(pA), bb = ballot(pB);
                 const int ca = __popcll(ba), cb = __popcll(bb);
                 if (navail + ca + cb > cap) {
@@ -882,10 +869,9 @@ __device__ __noinline__ int wide_run(PackLds* L, int h, const int* abort_flag, i
             S.status = status;
             S.used = navail;
             S.dif = dif;
-        }
+        } else if (many) L->many = 1;
     }
     wave_sync();
-    return many;
 }
 
 // ---- between passes ------------------------------------------------------------------
@@ -1097,10 +1083,10 @@ static __device__ __noinline__ void pass_begin(PackLds* L, int h)
     wave_sync();
 }
 
-// The trace points that the paths in the PackBands have already are done;
-// whether there were any.
+// The trace points that the paths in the PackBands have already are done.
+// many: whether there were any, so that the next wave looks again.
 template <int NCH>
-__device__ __noinline__ bool pack_skip(PackLds* L)
+__device__ __noinline__ void pack_skip(PackLds* L)
 {
     const int lane = __lane_id(), sl = lane & 31;
     const PackSlot& S = L->slot[lane >> 5];
@@ -1115,26 +1101,26 @@ __device__ __noinline__ bool pack_skip(PackLds* L)
     Glob<Int4>* pool = (Glob<Int4>*)S.pool;
     if (fA) D.tA[sl] = skip_points(pool, D.HA[sl], tA, TS, 0, m);
     if (fB) D.tB[sl] = skip_points(pool, D.HB[sl], tB, TS, offB, m);
+    if (lane == 0) L->many = 0;
+    if (any_lane(fA || fB) && lane == 0) L->many = 1;
     wave_sync();
-    return any_lane(fA || fB);
 }
 
 // The halves in `stopped` (bit 0: lanes 0..31): a pass that needs the wave
 // gets it, one that ended is followed by the next.  Afterwards every slot
 // holds a pass that goes on from its PackBand, or is idle with an empty band.
-// kMany in `stopped`, or from wide_run: pack_skip.  Returns kMany where the next wave needs it again.
 template <int NCH, class Job>
-__device__ __noinline__ unsigned pack_serve(Job job, PackLds* L, unsigned stopped, const int* abort_flag)
+__device__ __noinline__ void pack_serve(Job job, PackLds* L, unsigned stopped, const int* abort_flag)
 {
     const int lane = __lane_id();
-    int many = (stopped & kMany) ? 1 : 0;
+    stopped = (unsigned)uni((int)stopped);
     for (int h = 0; h < 2; h++) {
         if (!((stopped >> h) & 1)) continue;
         PackSlot& S = L->slot[h];
         bool go = false;
         for (;;) {
             if (uni(S.phase) != PH_IDLE && uni(S.status) == LA_GROW) {
-                many |= uni(wide_run<NCH>(L, h, abort_flag, many));
+                wide_run<NCH>(L, h, abort_flag);
                 go = uni(S.running) != 0;
                 if (lane == 0) {
                     S.running = 0;
@@ -1160,7 +1146,7 @@ __device__ __noinline__ unsigned pack_serve(Job job, PackLds* L, unsigned stoppe
         }
     }
     set_priority(max(uni(L->slot[0].prio), uni(L->slot[1].prio)));
-    return many && pack_skip<NCH>(L) ? kMany : 0;
+    if (uni(L->many)) pack_skip<NCH>(L);
 }
 
 // ---- the loop --------------------------------------------------------------------------
@@ -1227,7 +1213,8 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
                 }
             }
             wave_sync();
-            stopped = (unsigned)uni((int)pack_serve<NCH>(job, &L, stopped, abort_flag));
+            pack_serve<NCH>(job, &L, stopped, abort_flag);
+            stopped = uni(L.many) ? kMany : 0;
             lane = __lane_id();
 #ifndef MI_CPU_WAVE_EMU
             asm volatile("" : "+v"(lane));   // computed here, not once before the loop
@@ -1286,7 +1273,8 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
             int nA = point_at<NCH>(tA, TS), nB = point_at<NCH>(tB, TS) + offB;
             const Lanes in = ballot(sl >= a) & ballot(sl <= b);
             Lanes wA = in & ballot(x >= nA), wB = in & ballot(y >= nB);
-            if (wA | wB) for (int n = 1;; n++) {   // n: points passed
+            int n = 0;   // points passed
+            while (wA | wB) {
                 const Lanes pA = wA & (fresh | ballot((int)(((unsigned)tA << 24) - ((unsigned)HA & ~(unsigned)kPebIdx)) > 0));
                 const Lanes pB = wB & (fresh | ballot((int)(((unsigned)tB << 24) - ((unsigned)HB & ~(unsigned)kPebIdx)) > 0));
                 const int al = __popcll(pA & 0xffffffffull), bl = __popcll(pB & 0xffffffffull);
@@ -1310,8 +1298,11 @@ __device__ __forceinline__ void pack_run(PackLds& L, Job job, bool second, const
                 nB = point_at<NCH>(tB, TS) + offB;
                 wA &= ballot(x >= nA);
                 wB &= ballot(y >= nB);
-                if (!(wA | wB)) break;
-                if (n == kManyPoints - 1) stopped = kMany;
+                n++;
+            }
+            if (n >= kManyPoints) {
+                stopped = kMany;
+                L.many = 1;
             }
         }
 
