@@ -519,8 +519,8 @@ def main():
                                "note": "one step whose index build uploads the block's reads from host memory"},
             "roofline": {"bound": "valu", "kernel": "k_report (two read pairs per wave64: gating + Local_Alignment)",
                          "achieved": round(ach, 2), "peak": VALU_PEAK_GOPS, "unit": "Gop/s (W_align lane-ops)",
-                         "frac": round(ach / VALU_PEAK_GOPS, 5), "traffic": profiled_traffic("k_report<1, false>"),
-                         "traffic_unit": "HBM bytes per launch of the one-alignment-per-wave k_report (rocprofv3 --pmc, calibrated)",
+                         "frac": round(ach / VALU_PEAK_GOPS, 5), "traffic": profiled_traffic("k_report<2, false>"),
+                         "traffic_unit": "HBM bytes per k_report<2, false> launch (rocprofv3 --pmc, calibrated)",
                          "kernel_ms_per_step": round(k_report * 1e3, 2), "launches_per_step": launches,
                          "w_align_per_step": w_align, "issue": issue},
             "roofline_hbm": {"bound": "hbm", "kernel": "seed LSD radix sort (rs_hist + rs_scatter)",

@@ -37,8 +37,8 @@
 //   * What only changes at events lives in LDS, written by the lane that owns
 //     the event: the trim point, the best point's y, the boundary point.
 //
-// What bounds it, on a full GPU: VALU issue -- 2.66e10 wave64 VALU
-// instructions per report launch on the 5 Mbp / 30x block (196 per step of two
+// What bounds it, on a full GPU: VALU issue -- 2.65e10 wave64 VALU
+// instructions per report launch on the 5 Mbp / 30x block (195 per step of two
 // alignments), 43 ms of the 45 ms it takes at one per SIMD every 4 cycles; one
 // alignment per wave needed 5.2e10 and 96 ms (and 6.6 ms more for the pairs
 // wider than 64 diagonals, run again at 128).  So the sets of lanes are kept as

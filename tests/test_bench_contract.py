@@ -25,7 +25,7 @@ def test_more_than_one_gpu_exits_with_a_message():
 
 def test_profiled_traffic_reads_the_committed_counters():
     b = _bench()
-    rep = b.profiled_traffic("k_report<1, false>")
+    rep = b.profiled_traffic("k_report<2, false>")
     hist, scat = b.profiled_traffic("rs_hist<Seed>"), b.profiled_traffic("rs_scatter<Seed>")
     # calibrated bytes per launch: 2 x FETCH_SIZE KiB + WRITE_SIZE KiB
     assert rep is not None and 5e9 < rep < 5e10
