@@ -48,7 +48,7 @@
 // wait for LDS).  Where few alignments are left (repeat-rich
 // blocks: one pair with 90 alignments one after another, 55 % of the CUs busy
 // over the launch) it is the latency of one wave's step, about 1.5 us.
-// Waves per SIMD, ms a pass against 6 in turn on one box:
+// Waves per SIMD, ms a pass against 6 (both in turn on one GPU):
 //   4: 5 Mbp block 186 : 179, repeat-rich 201 : 207, 400,000 tasks that start
 //      off their diagonal 54.2 : 48.4, 20,000 tasks 19.2 : 21.8
 //   5: 197 : 189, 254 : 259, 50.6 : 49.1, 19.8 : 21.6

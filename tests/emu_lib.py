@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import ctypes as C
+import fcntl
 import os
 import subprocess
 from contextlib import contextmanager
@@ -14,7 +15,9 @@ HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "wave_emu")
 
 
 def build():
-    subprocess.check_call(["make", "-s", "-j2", "-C", HERE, "libs"])
+    with open(os.path.join(HERE, ".lock"), "w") as f:   # one builder at a time (pytest -n)
+        fcntl.flock(f, fcntl.LOCK_EX)
+        subprocess.check_call(["make", "-s", "-j2", "-C", HERE, "libs"])
 
 
 class Lib:
